@@ -119,4 +119,39 @@ __device__ __forceinline__ float exp2_rep_nonpos(float x) {
   return x > -125.0f ? r : 0.0f;
 }
 
+// Buffer resource over `bytes` bytes from `base` (raw: no stride, no
+// swizzle; word 3 the data format gfx9 parts take for untyped loads), and the
+// buffer load of 16 bytes per lane into LDS (lane l at lds + 16 l; M0 holds
+// the wave-uniform LDS base) at base + voffset + soffset.  Bytes at or past
+// `bytes` read as zeros.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ i32x4 buffer_rsrc(const void* base, unsigned bytes) {
+  const unsigned long long a = reinterpret_cast<unsigned long long>(base);
+  i32x4 r;
+  r[0] = (int)(unsigned)a;
+  r[1] = (int)(unsigned)(a >> 32);
+  r[2] = (int)bytes;
+  r[3] = 0x00020000;
+  return r;
+}
+// The same over fp16 data for raw_buffer_load_format4, which loads four halves
+// (8-byte aligned offset) and returns them converted to fp32: destination
+// x, y, z, w, number format float, data format 16_16_16_16.
+__device__ __forceinline__ i32x4 buffer_rsrc_f16x4(const void* base, unsigned bytes) {
+  i32x4 r = buffer_rsrc(base, bytes);
+  r[3] = 4 | (5 << 3) | (6 << 6) | (7 << 9) | (7 << 12) | (12 << 15);
+  return r;
+}
+__device__ f32x4 raw_buffer_load_format4(i32x4 rsrc, int voffset, int soffset, int aux)
+    __asm("llvm.amdgcn.raw.buffer.load.format.v4f32");
+__device__ void raw_buffer_load_lds(i32x4 rsrc, __attribute__((address_space(3))) unsigned* lds, int size,
+                                    int voffset, int soffset, int offset, int aux)
+    __asm("llvm.amdgcn.raw.buffer.load.lds");
+__device__ __forceinline__ void buffer_load_lds16(i32x4 rsrc, __attribute__((address_space(3))) unsigned* lds,
+                                                  unsigned voffset, int soffset) {
+  raw_buffer_load_lds(rsrc, lds, 16, (int)voffset, soffset, 0, 0);
+}
+__device__ i32x4 raw_buffer_load_b128(i32x4 rsrc, int voffset, int soffset, int aux)
+    __asm("llvm.amdgcn.raw.buffer.load.v4i32");
+
 }  // namespace qd

@@ -208,8 +208,6 @@ struct BatchedGemvParams {
   // Joint gate/up form only (launch_gemm_mfma_swiglu): W2, the up weight, with
   // w as W1 and y = act.
   const uint16_t* w2;
-  // Exact two-row form only: tokens per workgroup (0: 32); set by launch_gemv_batched.
-  int tok_per_wg = 0;
 };
 
 // Causal prefill attention of `tokens` queries at positions pos0, pos0 + 1, ...
@@ -376,6 +374,10 @@ hipError_t launch_lm_head_argmax(const LmHeadParams& p, int* token, hipStream_t 
 hipError_t launch_rmsnorm_batched(const uint16_t* x, const uint16_t* w, float eps, uint16_t* xn,
                                   int hidden, int T, hipStream_t stream);
 hipError_t launch_gemv_batched(const BatchedGemvParams& p, int epi, hipStream_t stream);
+// The same on the fp32 matrix instructions (qd_exact_gemm.hip), for `cus` compute
+// units; launch_gemv_batched says when.  p.ldx below 2^26, fewer than 2^20 tiles
+// of 32 x 32 outputs.
+hipError_t launch_gemm_exact_mfma(const BatchedGemvParams& p, int epi, int cus, hipStream_t stream);
 // The same product on the matrix cores (fp32 accumulation in the hardware's
 // order, not bit-reproducible on the host); p.k must be a multiple of 64.
 hipError_t launch_gemm_mfma(const BatchedGemvParams& p, int epi, hipStream_t stream);

@@ -65,6 +65,76 @@ def test_exact_mode_is_the_decode_gemv(qdiy, m, n, k, with_res):
         assert _same(got[i], want), f"row {i}"
 
 
+@pytest.mark.parametrize("m,n,k", [
+    # the two-row kernel's last token count and the matrix instructions' first
+    (4, 33, 72), (5, 33, 72),
+    # edges of the 16 x 16 and 32 x 32 output tiles in both directions
+    (15, 16, 512), (16, 17, 520), (17, 31, 1032), (31, 33, 1000), (33, 32, 2056), (65, 65, 64),
+    # K: one class, a group of classes partly filled, whole groups without a last
+    # chunk, the widest (from one token on the matrix instructions)
+    (9, 40, 8), (40, 40, 440), (70, 48, 1536), (3, 40, 8192), (100, 50, 7176),
+    # 32 x 32 tiles: several rounds of a device's workgroups
+    (520, 1100, 136)])
+@pytest.mark.parametrize("with_res", [False, True])
+def test_exact_mode_tile_edges(qdiy, m, n, k, with_res):
+    """Every output of the exact mode where its tiles, its last chunk of K or its
+    choice of kernel change, bit for bit; x and y rows padded, y at an odd element
+    offset (no 8-byte stores) without a residual."""
+    rng = np.random.default_rng(m * 77 + n + k + with_res)
+    ldx, ldy, off = k + 8, n + (4 if with_res else 3), 0 if with_res else 1
+    x, W = normal_f16(rng, (m, ldx)), normal_f16(rng, (n, k), 0.02)
+    R = normal_f16(rng, (m, ldy))
+    y = torch.full((off + m * ldy + 8,), 9.0, dtype=torch.float16, device="cuda")
+    qdiy.gemm_nt(_dev(x.reshape(-1)), _dev(W.reshape(-1)), y[off:], m, n, k, ldx=ldx, ldy=ldy,
+                 residual=_dev(R.reshape(-1)) if with_res else None, mode=qdiy.GEMM_EXACT)
+    torch.cuda.synchronize()
+    out = y.cpu().numpy()
+    got = out[off:off + m * ldy].reshape(m, ldy)
+    assert np.all(got[:, n:] == np.float16(9.0)) and np.all(out[:off] == 9.0) and np.all(out[off + m * ldy:] == 9.0)
+    for i in range(m):
+        if with_res:
+            want = oracle.proj_residual(x[i, :k], W.reshape(-1), R[i, :n], n, k)
+        else:
+            want = oracle.gemv(x[i, :k], W.reshape(-1), n, k, 0, oracle.ORDER_WAVE64)
+        assert _same(got[i, :n], want), f"row {i}"
+
+
+def test_exact_mode_infinities_stay_in_their_row(qdiy):
+    """An infinity in one token's or weight's row (next to the last chunk, whose elements
+    past K belong to the following row) reaches that row's outputs only, with the
+    oracle's infinities and NaNs."""
+    m, n, k = 40, 48, 456
+    rng = np.random.default_rng(5)
+    x, W = normal_f16(rng, (m, k)), normal_f16(rng, (n, k), 0.02)
+    x[7, 0], x[20, k - 1], W[33, 0], W[11, 448] = np.inf, -np.inf, np.inf, np.nan
+    y = torch.zeros(m * n, dtype=torch.float16, device="cuda")
+    qdiy.gemm_nt(_dev(x.reshape(-1)), _dev(W.reshape(-1)), y, m, n, k, mode=qdiy.GEMM_EXACT)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().reshape(m, n)
+    with np.errstate(invalid="ignore"):
+        want = np.stack([oracle.gemv(x[i], W.reshape(-1), n, k, 0, oracle.ORDER_WAVE64) for i in range(m)])
+    nan = np.isnan(want)
+    assert np.array_equal(np.isnan(got), nan) and nan.any() and np.isinf(want).any()
+    assert np.array_equal(got.view(np.uint16)[~nan], want.view(np.uint16)[~nan])
+
+
+def test_exact_mode_far_apart_rows(qdiy):
+    """Token rows 2^26 elements apart, beyond the matrix kernel's 32-bit lane offsets,
+    take the two-row kernel: the same bits."""
+    m, n, k, ldx = 6, 64, 264, 1 << 26
+    rng = np.random.default_rng(6)
+    x, W = normal_f16(rng, (m, k)), normal_f16(rng, (n, k), 0.02)
+    far = torch.empty((m - 1) * ldx + k, dtype=torch.float16, device="cuda")
+    for i in range(m):
+        far[i * ldx:i * ldx + k] = _dev(x[i])
+    y = torch.zeros(m * n, dtype=torch.float16, device="cuda")
+    qdiy.gemm_nt(far, _dev(W.reshape(-1)), y, m, n, k, ldx=ldx, mode=qdiy.GEMM_EXACT)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().reshape(m, n)
+    for i in range(m):
+        assert _same(got[i], oracle.gemv(x[i], W.reshape(-1), n, k, 0, oracle.ORDER_WAVE64)), f"row {i}"
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 64, 64), (37, 100, 512), (127, 6144, 2048), (256, 2048, 5504),
                                    (200, 5504, 2048),
                                    # from 128 rows: the 64 x 64 tile where a 128 x 128 grid would
