@@ -538,6 +538,413 @@ __global__ __launch_bounds__(NW * 64) void decode_attention_scan_kernel(AttnPara
   }
 }
 
+// ---------------------------------------------------------------------------
+// Exact prompt attention on the fp32 matrix instructions: 16 consecutive
+// queries share the rows they read.
+//
+// A batched query does, bit for bit, what the scan kernel does for it: the rows
+// of its plan's split c go to waves and 16-lane groups by its tiles, each group
+// keeps (m, l, O), and the groups, waves and splits fold in their fixed
+// orders.  None of that depends on the query except where its rows end, so
+// queries of one plan (64 consecutive lengths at 16 heads) can share every
+// load, and with 16 of them the two products are matrix products.
+// v_mfma_f32_16x16x1_4b_f32 adds one product per sum, rounded once
+// (qd_exact_gemm.hip; checked the same way with subnormal products and sums), and
+// its four blocks are the four groups:
+//   * scores, S^T = K Q^T: block b of quad qd adds the 8 products of dims 8 t ..
+//     8 t + 7, t = 4 qd + b, which is lane t's chain of dot8, and the 16 sums
+//     are added in row16_sum's tree.  (dot8 starts from -0, these sums from +0: a
+//     score's zero may change its sign, which no exponential sees.)  The A rows
+//     are ordered so that lane l receives, for query l % 16, the four rows of
+//     group l / 16: every softmax step is one lane's own, with no exchange;
+//   * O: step u multiplies group b's row u of V by the queries' weights in block
+//     b; lane l's own weight is the A operand, its 16 bytes of V's row (dims 8 j
+//     .. 8 j + 7, j = l % 16) the B operands of eight products.
+// Only the rescale and the fold of the groups pass values between lanes (the 4
+// groups' factors of 16 queries, through LDS).
+//
+// What bounds it: the scan alone read every query's K/V rows from L2 (9 TB/s
+// over the device at 16 heads) and spent 217 instructions per 16 rows of one
+// query; here 16 rows x 16 queries take 64 MFMAs (2048 cycles) and ~600 other
+// vector instructions, which share the same units, and half the time of a
+// workgroup's short life (16 rows per wave up to 1024 rows) is its first loads,
+// its folds and its end.  16 heads, whole calls: 256 queries from row 768 on
+// 171 -> 65 us (14 of it the merge kernel), from 2000 472 -> 105, from 5000
+// 1400 -> 263; 127 queries from row 0 16.6 -> 10 us.
+//
+// A wave takes 16 rows at a time: one tile of 4-row groups (U = 4) or two
+// consecutive ones of 2-row groups.  NW is the plan's waves (the order of the
+// sums), PW the waves that run; each of those takes the plan's waves w, w + PW,
+// ...  Rows past a query's end score -inf and their weight is 0, as in the
+// scan; there the scan multiplies it by the query's own last row, this kernel by
+// the row itself, which is the same for any finite V.  So where the block's
+// queries end in different rows, those rows of V are looked at first, and if
+// one holds an infinity or a NaN the block takes the scan's own steps.
+// kSplit: the split's partials, in the batched scan's slots; else (fused plans)
+// the outputs.
+constexpr int kPfQ = 16;                       // queries per workgroup
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+template <int NW>
+struct PrefillLds {
+  float so[NW][kPfQ][kD];
+  float sm[NW][kPfQ];
+  float sl[NW][kPfQ];
+  f32x4 alpha[NW][kPfQ];                       // a wave's rescale by query and group,
+  f32x4 factor[NW][kPfQ];                      // and its groups' factors in their fold
+  f32x4 q[kPfQ][kD / 4];                       // fp32, piece i of query r at i ^ (r % 8): no bank conflicts
+};
+
+// The scan's own steps for queries lo .. hi over split c, one after another
+// (each of the plan's waves on one of the PW that run).
+template <int NW, int PW, int U, bool kSplit>
+__device__ __forceinline__ void scan_queries(const AttnParams& p, PrefillLds<NW>& lds, int h, int c, int lo,
+                                                       int hi, int rows, int splits, bool inter) {
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int t = lane & 15, g = lane >> 4;
+  const int r0 = inter ? 0 : c * rows;
+  const long long off = h * p.head_stride + (long long)r0 * p.row_stride;
+  const char* const kb = reinterpret_cast<const char*>(p.k + off);
+  const char* const vb = reinterpret_cast<const char*>(p.v + off);
+  for (int L = lo; L <= hi; ++L) {
+    if (!inter && r0 >= L) continue;
+    const int b = L - p.seqlen;
+    const int n = inter ? interleaved_rows(L, NW * 4 * U, splits, c) : min(L - r0, rows);
+    const f16x8 qv = *reinterpret_cast<const f16x8*>(p.q + b * p.q_batch_stride + h * kD + t * 8);
+    for (int w = wave; w < NW; w += PW) {
+      GroupState st;
+      init_state(st);
+      if (inter)
+        scan_rows<NW, U, 1, true>(st, kb, vb, (unsigned)(p.row_stride * 2), n, w, g, t, qv, p.scale_log2, c, splits);
+      else
+        scan_rows<NW, U, 1, false>(st, kb, vb, (unsigned)(p.row_stride * 2), n, w, g, t, qv, p.scale_log2);
+      wave_merge(st);
+      if (lane < 16) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) lds.so[w][0][t * 8 + e] = st.o[e];
+        if (t == 0) {
+          lds.sm[w][0] = st.m;
+          lds.sl[w][0] = st.l;
+        }
+      }
+    }
+    __syncthreads();
+    if (tid < kD) {
+      float M = -__builtin_inff(), Ls = 0.0f, O = 0.0f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) M = fmaxf(M, lds.sm[w][0]);
+      const float base = safe_base(M);
+#pragma unroll
+      for (int w = 0; w < NW; ++w) {
+        const float wt = exp2_rep_nonpos(lds.sm[w][0] - base);
+        Ls = __builtin_fmaf(wt, lds.sl[w][0], Ls);
+        O = __builtin_fmaf(wt, lds.so[w][0][tid], O);
+      }
+      if constexpr (kSplit) {
+        const long long slot = ((long long)b * p.num_heads + h) * p.split_stride + c;
+        p.part_o[slot * kD + tid] = O;
+        if (tid == 0) p.part_ml[slot] = float2{M, Ls};
+      } else {
+        reinterpret_cast<_Float16*>(p.out + b * p.out_batch_stride)[h * kD + tid] = to_f16(O / Ls);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// The queries of rows lo .. hi (one plan, at most 16, in the block from row
+// first on) over split c: the contiguous rows from c * rows on, or interleaved
+// blocks of NW * 4 * U rows (inter) dealt over `splits`.  kOne: no wave has more
+// than 16 rows; then O is formed in two halves of the dims, whose 64 registers
+// leave room for three waves per SIMD instead of two (the loads, the Q rows and
+// the fold of a workgroup's short life overlap with other workgroups only).
+template <int NW, int PW, int U, bool kSplit, bool kOne>
+__device__ __forceinline__ void prefill_block(const AttnParams& p, PrefillLds<NW>& lds, int h, int c,
+                                              int first, int lo, int hi, int rows, int splits, bool inter) {
+  constexpr int kStep = NW * 4 * U;            // rows from one of a wave's tiles to its next
+  constexpr int kTiles = 4 / U;                // tiles per 16 rows
+  constexpr int kND = kOne ? 4 : 8;            // products (dims 8 ql + n) of O at a time
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ql = lane & 15, g = lane >> 4;
+  const unsigned row_bytes = (unsigned)(p.row_stride * 2);
+  const char* const kb = reinterpret_cast<const char*>(p.k + h * p.head_stride);
+  const char* const vb = reinterpret_cast<const char*>(p.v + h * p.head_stride);
+  // rows of the split that a query over L rows sees, and the split's j-th row
+  auto rows_of = [&](int L) {
+    return inter ? interleaved_rows(L, kStep, splits, c) : max(0, min(L - c * rows, rows));
+  };
+  auto layer_row = [&](int j) {
+    return !kOne && inter ? (unsigned)(((j / kStep) * splits + c) * kStep + (j & (kStep - 1)))
+                          : (unsigned)(c * rows + j);
+  };
+  // row rr (0..3) of group gi among the 16 rows from tile row blk on
+  auto row_at = [&](int blk, int gi, int rr) {
+    return blk + gi + (U == 4 ? 4 * rr : (rr >> 1) * kStep + 4 * (rr & 1));
+  };
+  const int nmax = rows_of(hi), nmin = rows_of(lo);
+  // 16 rows of K (lane: row ql's dims 8 (4 qd + g) .. + 8) and V (lane: its
+  // group's rows, dims 8 ql .. + 8), rows past the last clamped to it.
+  f16x8 kr[4], vr[4];
+  auto load = [&](int blk) {
+    const unsigned ko = layer_row(min(row_at(blk, ql >> 2, ql & 3), nmax - 1)) * row_bytes + 16u * g;
+#pragma unroll
+    for (int qd = 0; qd < 4; ++qd) kr[qd] = *reinterpret_cast<const f16x8*>(kb + (ko + 64u * qd));
+#pragma unroll
+    for (int rr = 0; rr < 4; ++rr)
+      vr[rr] = *reinterpret_cast<const f16x8*>(
+          vb + (layer_row(min(row_at(blk, g, rr), nmax - 1)) * row_bytes + 16u * ql));
+  };
+  if (wave * 4 * U < nmax) load(wave * 4 * U); // ahead of all that is waited for
+  const int L = first + ql;
+  const int n_q = L >= lo && L <= hi ? rows_of(L) : 0;
+  int bad = 0;
+  if (tid < 256) {                             // query tid / 16's dims 8 ql .. + 8
+    const int r = tid >> 4;
+    const uint16_t* q = p.q + (long long)(min(max(first + r, lo), hi) - p.seqlen) * p.q_batch_stride + h * kD;
+    const f16x8 v = *reinterpret_cast<const f16x8*>(q + 8 * ql);
+    if (nmin != nmax) {                        // at most 16 rows: from the first query's last one on
+      const int j = nmin - 1 + r;
+      if (j >= 0 && j < nmax) {
+        const auto w = *reinterpret_cast<const i32x4*>(vb + (layer_row(j) * row_bytes + 16u * ql));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          bad |= ((w[i] & 0x7c00) == 0x7c00) | ((w[i] & 0x7c000000) == 0x7c000000);
+      }
+    }
+    lds.q[r][(2 * ql) ^ (r & 7)] = f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+    lds.q[r][(2 * ql + 1) ^ (r & 7)] = f32x4{(float)v[4], (float)v[5], (float)v[6], (float)v[7]};
+  }
+  if (__syncthreads_or(bad)) {
+    scan_queries<NW, PW, U, kSplit>(p, lds, h, c, lo, hi, rows, splits, inter);
+    return;
+  }
+
+  for (int w = wave; w < NW; w += PW) {
+    float m = -__builtin_inff(), l = 0.0f;
+    float s[4];                                // the lane's query's scores of its group's rows, then weights
+    auto scores = [&](int blk) {
+      f32x4 sum = {}, part = {};
+#pragma unroll
+      for (int qd = 0; qd < 4; ++qd) {
+        f32x16 a = {};
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {       // dims 8 (4 qd + g) + 4 hf .. + 4
+          const f32x4 qa = lds.q[ql][(8 * qd + 2 * g + hf) ^ (ql & 7)];
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            a = __builtin_amdgcn_mfma_f32_16x16x1f32((float)kr[qd][4 * hf + e], qa[e], a, 0, 0, 0);
+        }
+        f32x4 t;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t[r] = (a[r] + a[4 + r]) + (a[8 + r] + a[12 + r]);
+        if (qd == 0 || qd == 2) part = t;
+        if (qd == 1) sum = part + t;
+        if (qd == 3) sum = sum + (part + t);
+        __builtin_amdgcn_sched_barrier(0);     // (else conversions go first, and registers run out)
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s[r] = row_at(blk, g, r) < n_q ? sum[r] * p.scale_log2 : -__builtin_inff();
+    };
+    // One tile's softmax step: s becomes the weights; returns the rescale.
+    auto softmax = [&](int tl) {
+      float mt = s[tl * U];
+#pragma unroll
+      for (int u = 1; u < U; ++u) mt = fmaxf(mt, s[tl * U + u]);
+      const float mn = fmaxf(m, mt);
+      const float base = safe_base(mn);
+      const float alpha = exp2_rep_nonpos(m - base);
+      l *= alpha;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        s[tl * U + u] = exp2_rep_nonpos(s[tl * U + u] - base);
+        l += s[tl * U + u];
+      }
+      m = mn;
+      return alpha;
+    };
+    // O[n][4 b + r]: group b, query 4 g + r, dim 8 ql + d0 + n
+    f32x16 O[kND];
+    auto rescale = [&](const f32x4 (&factor)[kPfQ]) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const f32x4 al = factor[4 * g + r];
+#pragma unroll
+        for (int n = 0; n < kND; ++n)
+#pragma unroll
+          for (int b = 0; b < 4; ++b) O[n][4 * b + r] *= al[b];
+      }
+    };
+    auto values = [&](int tl, int d0, bool start) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int n = 0; n < kND; ++n)
+          O[n] = __builtin_amdgcn_mfma_f32_16x16x1f32(s[tl * U + u], (float)vr[tl * U + u][d0 + n],
+                                                      start && u == 0 ? f32x16{} : O[n], 0, 0, 0);
+      }
+    };
+    // wave_merge's group sums (g0 + g1) + (g2 + g3) of the scaled O
+    auto put = [&](int d0) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const f32x4 f = lds.factor[w][4 * g + r];
+#pragma unroll
+        for (int n4 = 0; n4 < kND; n4 += 4) {
+          f32x4 o;
+#pragma unroll
+          for (int n = 0; n < 4; ++n)
+            o[n] = (O[n4 + n][r] * f[0] + O[n4 + n][4 + r] * f[1]) + (O[n4 + n][8 + r] * f[2] + O[n4 + n][12 + r] * f[3]);
+          *reinterpret_cast<f32x4*>(&lds.so[w][4 * g + r][8 * ql + d0 + n4]) = o;
+        }
+      }
+    };
+    // wave_merge's maximum, factor and sum
+    auto meet = [&] {
+      float M = fmaxf(m, __shfl_xor(m, 16));
+      M = fmaxf(M, __shfl_xor(M, 32));
+      const float sc = exp2_rep_nonpos(m - safe_base(M));
+      l *= sc;
+      l += __shfl_xor(l, 16);
+      l += __shfl_xor(l, 32);
+      if (g == 0) {
+        lds.sm[w][ql] = M;
+        lds.sl[w][ql] = l;
+      }
+      reinterpret_cast<float*>(&lds.factor[w][ql])[g] = sc;
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    };
+    int blk = w * 4 * U;
+    if (blk >= nmax) {                         // no rows: an empty state
+      meet();
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        *reinterpret_cast<f32x4*>(&lds.so[w][2 * i + (lane >> 5)][4 * (lane & 31)]) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      continue;
+    }
+    if (w != wave) load(blk);
+    if constexpr (kOne) {
+      scores(blk);
+      softmax(0);
+      const bool two = kTiles == 2 && blk + kStep < nmax;   // some query has the second tile
+      if (two) {
+        const float alpha = softmax(kTiles - 1);
+        reinterpret_cast<float*>(&lds.alpha[w][ql])[g] = alpha;
+      }
+      meet();
+#pragma unroll
+      for (int d0 = 0; d0 < 8; d0 += kND) {
+        values(0, d0, true);
+        if (two) {
+          rescale(lds.alpha[w]);
+          values(kTiles - 1, d0, false);
+        }
+        put(d0);
+      }
+    } else {
+      auto unit = [&](bool start) {
+        scores(blk);
+#pragma unroll
+        for (int tl = 0; tl < kTiles; ++tl) {
+          if (tl > 0 && blk + tl * kStep >= nmax) break;   // no query has this tile
+          const float m0 = m;
+          const float alpha = softmax(tl);
+          // as in the scan, the rescale changes no bit where no maximum rose
+          if (!(start && tl == 0) && __builtin_amdgcn_ballot_w64(m != m0)) {
+            reinterpret_cast<float*>(&lds.alpha[w][ql])[g] = alpha;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            rescale(lds.alpha[w]);
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          }
+          values(tl, 0, start && tl == 0);
+        }
+      };
+      unit(true);
+#pragma unroll 1
+      for (blk += kTiles * kStep; blk < nmax; blk += kTiles * kStep) {
+        load(blk);
+        __builtin_amdgcn_sched_barrier(0);
+        unit(false);
+      }
+      meet();
+      put(0);
+    }
+  }
+  __syncthreads();
+  // the waves' fold: thread (query, 8 dims)
+  const int q = tid >> 4;
+  const int Lq = first + q;
+  if (tid < 256 && Lq >= lo && Lq <= hi && (inter || c * rows < Lq)) {
+    float M = -__builtin_inff(), Ls = 0.0f, O[8] = {};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) M = fmaxf(M, lds.sm[w][q]);
+    const float base = safe_base(M);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float wt = exp2_rep_nonpos(lds.sm[w][q] - base);
+      Ls = __builtin_fmaf(wt, lds.sl[w][q], Ls);
+      const f32x4 a = *reinterpret_cast<const f32x4*>(&lds.so[w][q][8 * ql]);
+      const f32x4 b = *reinterpret_cast<const f32x4*>(&lds.so[w][q][8 * ql + 4]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        O[e] = __builtin_fmaf(wt, a[e], O[e]);
+        O[4 + e] = __builtin_fmaf(wt, b[e], O[4 + e]);
+      }
+    }
+    const int b = Lq - p.seqlen;
+    if constexpr (kSplit) {
+      const long long slot = ((long long)b * p.num_heads + h) * p.split_stride + c;
+      *reinterpret_cast<f32x4*>(p.part_o + slot * kD + 8 * ql) = f32x4{O[0], O[1], O[2], O[3]};
+      *reinterpret_cast<f32x4*>(p.part_o + slot * kD + 8 * ql + 4) = f32x4{O[4], O[5], O[6], O[7]};
+      if (ql == 0) p.part_ml[slot] = float2{M, Ls};
+    } else {
+      f16x8 o;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) o[e] = to_f16(O[e] / Ls);
+      *reinterpret_cast<f16x8*>(p.out + b * p.out_batch_stride + h * kD + 8 * ql) = o;
+    }
+  }
+}
+
+// Workgroup (split c, head h) = blockIdx.x as in the scan kernel; queries with
+// rows 16 y + 1 .. 16 y + 16 of those with p.seqlen .. p.seqlen + tokens - 1
+// rows, y counted from the first one's.  Where the 16 do not share a plan each
+// run of them that does is a block of its own.
+template <int NW, int PW, int U, bool kSplit, bool kOne>
+__global__ __launch_bounds__(PW * 64, kOne ? 3 : 2) void prefill_exact_kernel(AttnParams p, int tokens) {
+  __shared__ PrefillLds<NW> lds;
+  const int h = blockIdx.x % p.num_heads;
+  const int c = blockIdx.x / p.num_heads;
+  const int first = ((p.seqlen - 1) & ~(kPfQ - 1)) + 1 + kPfQ * blockIdx.y;
+  const int last = min(first + kPfQ, p.seqlen + tokens) - 1;
+  for (int lo = max(first, p.seqlen); lo <= last;) {
+    int splits = 1, rows = last, block = 0, hi = last;
+    if constexpr (kSplit) {
+      auto_plan(lo, p.num_cus, p.num_heads, p.long_inter != 0, &splits, &rows, &block);
+      auto same = [&](int n) {
+        int s1, r1, b1;
+        auto_plan(n, p.num_cus, p.num_heads, p.long_inter != 0, &s1, &r1, &b1);
+        return b1 == block && (block ? s1 == splits : r1 == rows);
+      };
+      // Once there is a split per CU the rows only grow with the length, and the
+      // last query tells for all; shorter ones are taken one by one.
+      if ((lo + kMinRowsPerSplit - 1) / kMinRowsPerSplit < p.num_cus / p.num_heads || !same(hi)) {
+        hi = lo;
+        while (hi < last && same(hi + 1)) ++hi;
+      }
+    }
+    if (block ? c < splits : c * rows < hi) {
+      prefill_block<NW, PW, U, kSplit, kOne>(p, lds, h, c, first, lo, hi, rows, splits, block != 0);
+      __syncthreads();                         // lds is free
+    }
+    lo = hi + 1;
+  }
+}
+
 // Stage 2: one workgroup per head folds the head's p.splits partials with the
 // log-sum-exp rule (fd_opt_stage2_kernel's role) and writes the fp16 output.
 // kBatch: workgroup (h, b = blockIdx.y) folds query b's auto_split partials
@@ -1311,19 +1718,53 @@ static void launch_scan_inter(const AttnParams& p, int waves, int rows_per_tile,
     hipLaunchKernelGGL((decode_attention_scan_kernel<4, 4, true, false, D, true>), grid, dim3(256), 0, stream, p);
 }
 
+// Whether a batched launch over `tokens` queries of p.seqlen rows on has them
+// share their rows (prefill_exact_kernel) or scans for each alone.  The shared
+// form's time is that of a block of 16 however few they are.  Kernel times, alone
+// / shared: fused plans 6.6 / 9.6 us at 32 queries, 8.2 / 9.0 at 48, 16.6 / 10 at
+// 127.  Split plans (with the merge; H heads, L rows) cross where H L tokens is
+// 60-100 thousand: H 16, L 300: 10.1 / 13.4 us at 8 queries, 14.7 / 13.5 at 16;
+// L 1000: 9.8 / 10.1 at 5, 13.9 / 10.2 at 8; H 8, L 600: 10.4 / 11.8 at 10, 15.3 /
+// 13.8 at 16; and from 4000 rows up at 6 queries (27.5 / 27.4 us: one block's
+// waves read a split's rows in turn).
+static bool prefill_shares_rows(const AttnParams& p, int tokens, bool split) {
+  if (!split) return tokens >= 56;
+  return tokens >= 6 && (long long)p.num_heads * p.seqlen * tokens >= 90000;
+}
+static unsigned prefill_blocks(const AttnParams& p, int tokens) {   // blocks of 16 lengths the queries touch
+  return (unsigned)((p.seqlen - 1 + tokens - 1) / kPfQ - (p.seqlen - 1) / kPfQ + 1);
+}
+
 hipError_t launch_decode_attention_fused_batch(const AttnParams& p, int tokens, hipStream_t stream) {
-  hipLaunchKernelGGL((decode_attention_scan_kernel<16, 4, false>), dim3(p.num_heads, tokens),
-                     dim3(16 * 64), 0, stream, p);
+  if (prefill_shares_rows(p, tokens, false)) {
+    hipLaunchKernelGGL((prefill_exact_kernel<16, 8, 4, false, true>), dim3(p.num_heads, prefill_blocks(p, tokens)),
+                       dim3(8 * 64), 0, stream, p, tokens);
+  } else {
+    hipLaunchKernelGGL((decode_attention_scan_kernel<16, 4, false>), dim3(p.num_heads, tokens),
+                       dim3(16 * 64), 0, stream, p);
+  }
   return hipGetLastError();
 }
 
-hipError_t launch_decode_attention_split_batch(const AttnParams& p, int rows_per_tile, int tokens,
+hipError_t launch_decode_attention_split_batch(const AttnParams& p, int rows_per_tile, bool one_tile, int tokens,
                                                hipStream_t stream) {
-  const dim3 scan_grid(p.num_heads * p.split_stride, tokens);
-  if (rows_per_tile == 4)
-    hipLaunchKernelGGL((decode_attention_scan_kernel<4, 4, true, true>), scan_grid, dim3(256), 0, stream, p);
-  else
-    hipLaunchKernelGGL((decode_attention_scan_kernel<4, 2, true, true>), scan_grid, dim3(256), 0, stream, p);
+  if (prefill_shares_rows(p, tokens, true)) {
+    const dim3 grid(p.num_heads * p.split_stride, prefill_blocks(p, tokens));
+    if (rows_per_tile == 4 && one_tile)
+      hipLaunchKernelGGL((prefill_exact_kernel<4, 4, 4, true, true>), grid, dim3(256), 0, stream, p, tokens);
+    else if (rows_per_tile == 4)
+      hipLaunchKernelGGL((prefill_exact_kernel<4, 4, 4, true, false>), grid, dim3(256), 0, stream, p, tokens);
+    else if (one_tile)
+      hipLaunchKernelGGL((prefill_exact_kernel<4, 4, 2, true, true>), grid, dim3(256), 0, stream, p, tokens);
+    else
+      hipLaunchKernelGGL((prefill_exact_kernel<4, 4, 2, true, false>), grid, dim3(256), 0, stream, p, tokens);
+  } else {
+    const dim3 scan_grid(p.num_heads * p.split_stride, tokens);
+    if (rows_per_tile == 4)
+      hipLaunchKernelGGL((decode_attention_scan_kernel<4, 4, true, true>), scan_grid, dim3(256), 0, stream, p);
+    else
+      hipLaunchKernelGGL((decode_attention_scan_kernel<4, 2, true, true>), scan_grid, dim3(256), 0, stream, p);
+  }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((decode_attention_merge_kernel<true>), dim3(p.num_heads, tokens),

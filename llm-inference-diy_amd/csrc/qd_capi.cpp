@@ -371,10 +371,12 @@ int attention_prefill(qd_ctx* ctx, const uint16_t* q, long long q_stride, const 
   }
   for (int t = n_fused; t < tokens;) {
     const qd::AttnPlan first = plan_auto(ctx, pos0 + t + 1);
+    // no wave of the plan's four has more than 16 rows
+    auto one_tile = [](const qd::AttnPlan& pl) { return !pl.block_rows && pl.rows_per_split <= 64; };
     int t1 = t + 1, max_splits = first.splits;
     for (; t1 < tokens && t1 - t < ctx->pf_tokens; ++t1) {
       const qd::AttnPlan pl = plan_auto(ctx, pos0 + t1 + 1);
-      if (pl.rows_per_tile != first.rows_per_tile) break;
+      if (pl.rows_per_tile != first.rows_per_tile || one_tile(pl) != one_tile(first)) break;
       max_splits = std::max(max_splits, pl.splits);
     }
     if (max_splits > ctx->pf_stride)
@@ -386,7 +388,7 @@ int attention_prefill(qd_ctx* ctx, const uint16_t* q, long long q_stride, const 
     p.part_ml = ctx->pf_part_ml;
     p.num_cus = ctx->num_cus;
     p.split_stride = max_splits;
-    const hipError_t e = qd::launch_decode_attention_split_batch(p, first.rows_per_tile, t1 - t, stream);
+    const hipError_t e = qd::launch_decode_attention_split_batch(p, first.rows_per_tile, one_tile(first), t1 - t, stream);
     if (e != hipSuccess) return hip_fail(e, "batched split attention launch");
     t = t1;
   }

@@ -140,6 +140,44 @@ def test_exact_mode_is_decode_attention(qdiy, H, pos0, T, layout, q_pad, out_pad
         pr.close()
 
 
+@pytest.mark.parametrize("H,pos0,T,layout", [
+    # fused plans in blocks of 16 queries: from an unaligned length, into split plans
+    (16, 3, 70, "engine"), (8, 57, 130, "head_major"),
+    # split plans of 16-row splits (queries of one block planned one by one), of 2-row
+    # and 4-row tiles with one and with several tiles per wave
+    (16, 129, 60, "engine"), (16, 700, 21, "engine"), (16, 950, 40, "head_major"), (4, 1400, 33, "engine"),
+    # head counts whose plans change inside a block of 16 lengths
+    (12, 500, 50, "engine"), (20, 830, 45, "engine"), (24, 300, 66, "head_major"), (32, 260, 40, "engine"),
+    # contiguous into interleaved 32-row blocks, and those into 64-row blocks
+    (16, 3050, 40, "engine"), (4, 3060, 26, "engine"), (8, 16370, 20, "engine")])
+@pytest.mark.parametrize("bad_v", [False, True])
+def test_exact_mode_shared_rows(qdiy, H, pos0, T, layout, bad_v):
+    """Queries that share their rows in blocks of 16: every one bit-identical to
+    qd_decode_attention at its length.  bad_v: infinities and NaNs in the last
+    queries' V rows and in one K row, which a query must see where it attends to the
+    row and nowhere else."""
+    pr = Prompt(qdiy, H, pos0, T, seed=H * 13 + pos0 + T + bad_v, layout=layout, q_pad=2 * H * D)
+    try:
+        if bad_v:
+            rng = np.random.default_rng(pos0 + T)
+            L = pos0 + T
+            hs, rs = (D, H * D) if layout == "engine" else (pr.kc.numel() // H, D)
+            for bad in (np.inf, -np.inf, np.nan):
+                for _ in range(3):
+                    j, h, d = int(rng.integers(max(0, L - 20), L)), int(rng.integers(H)), int(rng.integers(D))
+                    pr.vc[j * rs + h * hs + d] = float(bad)
+            pr.kc[(L - T // 2) * rs + 5] = float("inf")
+        got = pr.run(qdiy, qdiy.GEMM_EXACT)
+        want = pr.decode_rows(qdiy, range(T))
+        for t in range(T):
+            nan = np.isnan(want[t])
+            assert np.array_equal(np.isnan(got[t]), nan), f"query {t} (position {pos0 + t})"
+            assert _same(got[t][~nan], want[t][~nan]), f"query {t} (position {pos0 + t})"
+            assert bad_v or not nan.any()
+    finally:
+        pr.close()
+
+
 @pytest.mark.parametrize("H,pos0,T,layout,q_pad,out_pad",
                          CASES + [(16, 1792, 256, "engine", 4096, 0), (4, 0, 2048, "engine", 1024, 0),
                                   (16, 0, 2048, "engine", 4096, 0),      # a full pass at Qwen-1.8B's heads
