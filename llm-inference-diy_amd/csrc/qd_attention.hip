@@ -915,7 +915,7 @@ __device__ __forceinline__ void prefill_block(const AttnParams& p, PrefillLds<NW
 // rows, y counted from the first one's.  Where the 16 do not share a plan each
 // run of them that does is a block of its own.
 template <int NW, int PW, int U, bool kSplit, bool kOne>
-__global__ __launch_bounds__(PW * 64, kOne ? 3 : 2) void prefill_exact_kernel(AttnParams p, int tokens) {
+__global__ __launch_bounds__(PW * 64, kOne && PW == 4 ? 3 : 2) void prefill_exact_kernel(AttnParams p, int tokens) {
   __shared__ PrefillLds<NW> lds;
   const int h = blockIdx.x % p.num_heads;
   const int c = blockIdx.x / p.num_heads;

@@ -382,9 +382,9 @@ hipError_t launch_gemm_exact_mfma(const BatchedGemvParams& p, int epi, int cus, 
 // The same product on the matrix cores (fp32 accumulation in the hardware's
 // order, not bit-reproducible on the host); p.k must be a multiple of 64.
 hipError_t launch_gemm_mfma(const BatchedGemvParams& p, int epi, hipStream_t stream);
-// The same, allowed to split K over up to 8 slices when the tile grid leaves
-// CUs idle: fp32 partial sums in `workspace` (as many slices as it holds),
-// then one launch folds them in slice order and applies the epilogue.
+// The same, allowed to split K over two slices when the tile grid leaves half of
+// the CUs idle: fp32 partial sums in `workspace`, then one launch folds them in
+// slice order and applies the epilogue.
 // Otherwise, and without a workspace, it is launch_gemm_mfma.
 constexpr size_t kGemmSplitWsBytes = (size_t)64 << 20;
 hipError_t launch_gemm_mfma_split(const BatchedGemvParams& p, int epi, float* workspace,
@@ -392,8 +392,8 @@ hipError_t launch_gemm_mfma_split(const BatchedGemvParams& p, int epi, float* wo
 // act[t][i] = half(g * (u / (1 + exp(-u)))) with g = half(X W1^T), u = half(X W2^T)
 // (p.w = W1, p.w2 = W2, p.n = inter, p.y = act) in one matrix-core launch, the
 // SwiGLU applied in the GEMM's epilogue: from 128 tokens (act 8-byte aligned,
-// ldy a multiple of 4) the 192 x 256 or 128 x 128 ring tile, else the 64 x 64
-// tile.
+// ldy a multiple of 4) the 192 x 256 or 128 x 128 ring tile, else a short
+// prompt's.
 // hipErrorNotSupported (nothing launched) unless k is a multiple of 64: the
 // caller then runs the two projections and launch_swiglu_batched.
 hipError_t launch_gemm_mfma_swiglu(const BatchedGemvParams& p, hipStream_t stream);

@@ -387,9 +387,7 @@ __global__ __launch_bounds__(256) void embed_kernel(const uint16_t* __restrict__
 // would wait for every load in flight before each read.  Tiles past the last
 // repeat it, so every thread issues the same loads per stage and the wait
 // counts are fixed.  Tokens past t and rows past n load clamped rows and are
-// not stored.  K must be a multiple of 64.  kEpi 2 is the split-K form:
-// workgroup z = blockIdx.z sums K slice [z kslice, (z + 1) kslice) and stores
-// its fp32 tile to p.part.  kEpi 3 is the joint gate/up form: a workgroup
+// not stored.  K must be a multiple of 64.  kEpi 3 is the joint gate/up form: a workgroup
 // takes 32 intermediate rows, its W tile holding them from W1 (tile rows
 // 0..31) and W2 (32..63); wave w's B blocks are gate rows 16 (w % 2) .. +16
 // and the same up rows, so one lane holds g and u of the same output and writes
@@ -420,12 +418,7 @@ __global__ __launch_bounds__(256) void gemm_nt_mfma_kernel(BatchedGemvParams p) 
   const int wave = tid >> 6;
   const int n0 = blockIdx.x * (kEpi == 3 ? kMmTile / 2 : kMmTile);
   const int t0 = blockIdx.y * kMmTile;
-  int kbeg = 0, kend = p.k;
-  if constexpr (kEpi == 2) {
-    kbeg = blockIdx.z * p.kslice;
-    kend = min(p.k, kbeg + p.kslice);
-  }
-  const int ktiles = kend > kbeg ? (kend - kbeg) / kMmK : 0;
+  const int ktiles = p.k / kMmK;
 
   // Load i of wave w writes 1 KB at chunk 256 i + 64 w + lane of the stage's
   // operand: row 32 i + 8 w + lane / 8, position lane % 8.
@@ -435,11 +428,11 @@ __global__ __launch_bounds__(256) void gemm_nt_mfma_kernel(BatchedGemvParams p) 
   for (int i = 0; i < kMmOps; ++i) {
     const int row = 32 * i + 8 * wave + (lane >> 3);
     const int ch = (lane & 7) ^ mmswz(row);
-    xg[i] = p.x + (long long)min(t0 + row, p.t - 1) * p.ldx + kbeg + 8 * ch;
+    xg[i] = p.x + (long long)min(t0 + row, p.t - 1) * p.ldx + 8 * ch;
     if constexpr (kEpi == 3)
-      wg[i] = (row < 32 ? p.w : p.w2) + (long long)min(n0 + (row & 31), p.n - 1) * p.k + kbeg + 8 * ch;
+      wg[i] = (row < 32 ? p.w : p.w2) + (long long)min(n0 + (row & 31), p.n - 1) * p.k + 8 * ch;
     else
-      wg[i] = p.w + (long long)min(n0 + row, p.n - 1) * p.k + kbeg + 8 * ch;
+      wg[i] = p.w + (long long)min(n0 + row, p.n - 1) * p.k + 8 * ch;
   }
   auto issue = [&](int kt, MmStage& st) {
     const long long ko = (long long)min(kt, ktiles - 1) * kMmK;
@@ -546,10 +539,6 @@ __global__ __launch_bounds__(256) void gemm_nt_mfma_kernel(BatchedGemvParams p) 
       for (int r = 0; r < 4; ++r) {
         const int t = t0 + wm + 16 * i + (lane >> 4) * 4 + r;
         if (t >= p.t) continue;
-        if constexpr (kEpi == 2) {
-          p.part[((long long)blockIdx.z * p.t + t) * p.n + n] = acc[i][j][r];
-          continue;
-        }
         const _Float16 y = to_f16(acc[i][j][r]);
         _Float16* dst = reinterpret_cast<_Float16*>(p.y) + (long long)t * p.ldy + n;
         if constexpr (kEpi == 0) {
@@ -562,7 +551,7 @@ __global__ __launch_bounds__(256) void gemm_nt_mfma_kernel(BatchedGemvParams p) 
     }
 }
 
-// Folds the split-K partials of gemm_nt_mfma_kernel<2>: the slices' fp32 sums
+// Folds the split-K partials of gemm_nt_ring128_kernel<2>: the slices' fp32 sums
 // added in slice order, then the epilogue of kEpi (0: half(sum); 1: half(R +
 // half(sum))).  One thread per output.
 template <int kEpi>
@@ -580,7 +569,338 @@ __global__ __launch_bounds__(256) void splitk_fold_kernel(BatchedGemvParams p, i
 
 constexpr int kGemmXcds = 8;                 // MI355X: workgroups are dealt to 8 XCDs in turn
 constexpr int kRingMinRows = 128;            // the ring tiles from this many tokens
-constexpr int kGemmMaxSplits = 8;            // K slices of a split product
+
+// Short-prompt product: a workgroup computes 16 NB rows of W (outputs when kEpi
+// != 3) by 16 TB tokens, and its W waves share out K instead of the tile: wave w
+// multiplies the whole tile over K tiles w, w + W, ... of 64, staged through a ring
+// of S stages of its own (loaded straight into LDS; the rows' 16-byte chunks
+// swizzled as in gemm_nt_mfma_kernel).  No barrier until the waves' sums meet.
+//
+// Why: on gemm_nt_mfma_kernel's 64 x 64 tiles a 2048-row product of a short prompt
+// has 32 or 64 workgroups, each a chain of K / 64 barrier steps of ~0.24 us,
+// weights in L2 or not; 32 x 32 and 32 x 16 tiles have a workgroup for every CU and
+// eight chains in each.  What bounds them is the bytes each CU takes in: ~0.7 MB
+// per CU at 67 GB/s for K = 5504.  Cold weights, 100 tokens: 2048 x 2048 10.9 ->
+// 6.2 us, 2048 x 5504 26.5 -> 13.1; 16 tokens: 9.9 -> 5.6, 21.2 -> 13.3, 6144 x
+// 2048 10.3 -> 7.9 us.
+template <int NB, int TB, int W, int S, int kEpi>
+__global__ __launch_bounds__(64 * W, W / 4) void gemm_nt_wavek_kernel(BatchedGemvParams p) {
+  constexpr int kN = 16 * NB, kT = 16 * TB;             // rows of the W tile, tokens
+  constexpr int kOut = kEpi == 3 ? kN / 2 : kN;         // outputs per token
+  constexpr int kOps = (kN + kT) / 8;                   // 1 KB loads (8 rows of 128 bytes) per K tile
+  constexpr int kStage = (kN + kT) * 128;               // bytes
+  constexpr int kItems = NB * TB * 64;                  // f32x4 sums of the tile
+  __shared__ __align__(128) char lds[W][S * kStage];    // a wave's ring; at the end its sums
+  static_assert(kItems * 16 <= S * kStage, "a wave's sums fit its ring");
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ttiles = (p.t + kT - 1) / kT;
+  // XCD x takes a contiguous run of (W tile, token tile) pairs, token tile fastest
+  const int nwg = gridDim.x, xcd = blockIdx.x % kGemmXcds;
+  const int tile = xcd * (nwg / kGemmXcds) + min(xcd, nwg % kGemmXcds) + blockIdx.x / kGemmXcds;
+  const int n0 = (tile / ttiles) * kOut, t0 = (tile % ttiles) * kT;
+  const int ktiles = p.k / 64;
+  const int cnt = (ktiles - wave + W - 1) / W;          // this wave's K tiles (may be 0)
+
+  // Load i: rows 8 i .. + 8 of the tile (W's rows, W2's from kN / 2 in the gate/up
+  // form, then the tokens'), lane l row l / 8's chunk (l % 8) ^ (row % 8).  Rows past
+  // the operands read as zeros and feed only outputs that are not stored.
+  const int ch = (lane & 7) ^ (lane >> 3);
+  const unsigned wbytes = (unsigned)min(p.n - n0, kOut) * (unsigned)p.k * 2u;
+  const i32x4 rw = buffer_rsrc(p.w + (long long)n0 * p.k, wbytes);
+  const i32x4 rw2 = kEpi == 3 ? buffer_rsrc(p.w2 + (long long)n0 * p.k, wbytes) : rw;
+  const i32x4 rx = buffer_rsrc(p.x + (long long)t0 * p.ldx,
+                               (unsigned)(((long long)(min(p.t - t0, kT) - 1) * p.ldx + p.k) * 2));
+  unsigned voff[kOps];
+#pragma unroll
+  for (int i = 0; i < kOps; ++i) {
+    const unsigned row = 8 * i + (lane >> 3);
+    voff[i] = (row < kN ? (row % kOut) * (unsigned)p.k : (row - kN) * (unsigned)p.ldx) * 2u + 16u * ch;
+  }
+  char* const mine = lds[wave];
+  auto issue = [&](int j, int stage) {                  // this wave's j-th K tile; past the last: zeros
+    const int so = j < cnt ? (wave + W * j) * 128 : 0;
+#pragma unroll
+    for (int i = 0; i < kOps; ++i)
+      buffer_load_lds16(i >= kN / 8 ? rx : kEpi == 3 && i >= kN / 16 ? rw2 : rw,
+                        (__attribute__((address_space(3))) unsigned*)(mine + stage * kStage + 1024 * i),
+                        j < cnt ? voff[i] : 0x80000000u, so);
+  };
+  const int fr = lane & 15, fg = lane >> 4;
+  const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) char*)mine;
+  // step 0's chunk fg of row fr of block 0; blocks are 2048 bytes apart, step 1 at address ^ 64
+  const unsigned off = base + fr * 128 + 16 * (fg ^ (fr & 7));
+  f32x4_t acc[NB][TB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < TB; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  auto compute = [&](int stage, int refill) {
+    f16x8 f[2][NB + TB];
+    // this tile's loads: S - 1 newer tiles stay in flight
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * kOps) : "memory");
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < NB + TB; ++i)
+        asm volatile("ds_read_b128 %0, %1 offset:%2"
+                     : "=v"(f[ks][i]) : "v"((off ^ (64u * ks)) + stage * kStage), "n"(2048 * i) : "memory");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < NB + TB; ++i) asm volatile("" : "+v"(f[ks][i]));
+    issue(refill, stage);                               // the stage has been read
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < TB; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[ks][i], f[ks][NB + j], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int s = 0; s < S; ++s) issue(s, s);
+  int stage = 0;
+#pragma unroll 1
+  for (int j = 0; j < cnt; ++j) {
+    compute(stage, j + S);
+    stage = stage + 1 == S ? 0 : stage + 1;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // no load lands in the ring any more
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < TB; ++j) *reinterpret_cast<f32x4_t*>(mine + ((i * TB + j) * 64 + lane) * 16) = acc[i][j];
+  __syncthreads();
+  // item (block i, j, lane): rows n .. n + 3 of W for token t, four adjacent outputs
+  const bool vec = ((reinterpret_cast<uintptr_t>(p.y) | (kEpi == 1 ? reinterpret_cast<uintptr_t>(p.res) : 0)) & 7u) == 0 &&
+                   p.ldy % 4 == 0;
+  auto total = [&](int it) {
+    f32x4_t s = *reinterpret_cast<const f32x4_t*>(lds[0] + it * 16);
+#pragma unroll
+    for (int w = 1; w < W; ++w) s += *reinterpret_cast<const f32x4_t*>(lds[w] + it * 16);
+    return s;
+  };
+  for (int it = tid; it < (kEpi == 3 ? kItems / 2 : kItems); it += 64 * W) {
+    const int i = it / (64 * TB), j = it / 64 % TB;
+    const int t = t0 + 16 * j + fr, n = n0 + 16 * i + 4 * fg;
+    if (t >= p.t || n >= p.n) continue;
+    _Float16* dst = reinterpret_cast<_Float16*>(p.y) + (long long)t * p.ldy + n;
+    const f32x4_t a = total(it);
+    f16x4_t v;
+    if constexpr (kEpi == 3) {
+      const f32x4_t b = total(it + kItems / 2);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float gh = (float)to_f16(a[r]);
+        const float uh = (float)to_f16(b[r]);
+        const float e = exp2_rep(-uh * kLog2e);
+        v[r] = to_f16(gh * (uh / (1.0f + e)));
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = to_f16(a[r]);
+    }
+    const _Float16* res = reinterpret_cast<const _Float16*>(p.res) + (long long)t * p.ldy + n;
+    if (vec && n + 4 <= p.n) {
+      if constexpr (kEpi == 1) {
+        const f16x4_t rv = *reinterpret_cast<const f16x4_t*>(res);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = (_Float16)((float)rv[r] + (float)v[r]);
+      }
+      *reinterpret_cast<f16x4_t*>(dst) = v;
+    } else {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (n + r < p.n) dst[r] = kEpi == 1 ? (_Float16)((float)res[r] + (float)v[r]) : v[r];
+    }
+  }
+}
+
+// The same for wider tiles: KG groups of four waves (WW along W's rows, TW = 4 /
+// WW along the tokens, NB x TB blocks of 16 x 16 each) share out K, each group's
+// K tiles g, g + KG, ... going through a ring of S stages of its own, with one
+// barrier per K tile and the next tile's fragments read behind the products.
+// 64 x 128 tiles keep the gate and up rows of 100 tokens to one round of
+// workgroups (23.3 -> 18.3 us, 2 x 5504 x 2048; LDS reads and writes are ~0.5 of
+// the 0.6 us per K tile); 32 x 64 tiles fill the device for 48-64 tokens of 6144
+// rows (12.2-12.9 -> 10.2-10.9 us).
+template <int NB, int TB, int WW, int KG, int S, int kEpi>
+__global__ __launch_bounds__(256 * KG, KG) void gemm_nt_kgroup_kernel(BatchedGemvParams p) {
+  constexpr int TW = 4 / WW;
+  constexpr int kN = 16 * NB * WW, kT = 16 * TB * TW;
+  constexpr int kOut = kEpi == 3 ? kN / 2 : kN;
+  constexpr int kRows = kN + kT;
+  constexpr int kLoads = kRows / 32;                    // 1 KB loads per wave per K tile
+  constexpr int kStage = kRows * 128;
+  static_assert(kRows % 32 == 0 && kN % 32 == 0, "every wave the same loads of each operand");
+  static_assert(kEpi != 3 || (NB % 2 == 0 && kN % 64 == 0), "gate and up rows in pairs");
+  static_assert((KG - 1) * NB * TB * 4096 <= KG * S * kStage, "the groups' sums fit the rings");
+  __shared__ __align__(128) char lds[KG][S * kStage];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+  const int kg = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+  const int ttiles = (p.t + kT - 1) / kT;
+  const int nwg = gridDim.x, xcd = blockIdx.x % kGemmXcds;
+  const int tile = xcd * (nwg / kGemmXcds) + min(xcd, nwg % kGemmXcds) + blockIdx.x / kGemmXcds;
+  const int n0 = (tile / ttiles) * kOut, t0 = (tile % ttiles) * kT;
+  const int ktiles = p.k / 64;
+  const int iters = (ktiles + KG - 1) / KG;
+
+  // Load i of wave w: rows 32 i + 8 w .. + 8 of the tile
+  const int ch = (lane & 7) ^ (lane >> 3);
+  const unsigned wbytes = (unsigned)min(p.n - n0, kOut) * (unsigned)p.k * 2u;
+  const i32x4 rw = buffer_rsrc(p.w + (long long)n0 * p.k, wbytes);
+  const i32x4 rw2 = kEpi == 3 ? buffer_rsrc(p.w2 + (long long)n0 * p.k, wbytes) : rw;
+  const i32x4 rx = buffer_rsrc(p.x + (long long)t0 * p.ldx,
+                               (unsigned)(((long long)(min(p.t - t0, kT) - 1) * p.ldx + p.k) * 2));
+  unsigned voff[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const unsigned row = 32 * i + 8 * wave + (lane >> 3);
+    voff[i] = (row < kN ? (row % kOut) * (unsigned)p.k : (row - kN) * (unsigned)p.ldx) * 2u + 16u * ch;
+  }
+  char* const ring = lds[kg];
+  auto issue = [&](int it, int stage) {                 // the group's it-th K tile; past the last: zeros
+    const int kt = kg + KG * it;
+    const bool in = kt < ktiles;
+    const int so = in ? kt * 128 : 0;
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i)
+      buffer_load_lds16(i >= kN / 32 ? rx : kEpi == 3 && i >= kN / 64 ? rw2 : rw,
+                        (__attribute__((address_space(3))) unsigned*)(ring + stage * kStage + 4096 * i + 1024 * wave),
+                        in ? voff[i] : 0x80000000u, so);
+  };
+  const int wy = wave / TW, wx = wave % TW;
+  const int fr = lane & 15, fg = lane >> 4;
+  // tile row of block i of W, of block j of the tokens
+  auto wrow = [&](int i) {
+    return kEpi == 3 ? (i / (NB / 2)) * (kN / 2) + 8 * NB * wy + 16 * (i % (NB / 2)) : 16 * (NB * wy + i);
+  };
+  const unsigned base = (unsigned)(size_t)(__attribute__((address_space(3))) char*)ring;
+  unsigned addr[NB + TB];
+#pragma unroll
+  for (int i = 0; i < NB + TB; ++i)
+    addr[i] = base + (i < NB ? wrow(i) : kN + 16 * (TB * wx + i - NB)) * 128 + fr * 128 + 16 * (fg ^ (fr & 7));
+  typedef f16x8 Frags[2][NB + TB];
+  f32x4_t acc[NB][TB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int j = 0; j < TB; ++j) acc[i][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  auto read = [&](int stage, Frags& f) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < NB + TB; ++i)
+        asm volatile("ds_read_b128 %0, %1" : "=v"(f[ks][i]) : "v"((addr[i] ^ (64u * ks)) + stage * kStage) : "memory");
+  };
+  auto bind = [&](Frags& f) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < NB + TB; ++i) asm volatile("" : "+v"(f[ks][i]));
+  };
+  auto multiply = [&](const Frags& f) {
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < TB; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[ks][i], f[ks][NB + j], acc[i][j], 0, 0, 0);
+  };
+#pragma unroll
+  for (int s = 0; s < S; ++s) issue(s, s);
+  asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * kLoads) : "memory");
+  Frags fa, fb;
+  read(0, fa);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  bind(fa);
+  int stage = 0;
+  // Iteration it: tile it's fragments are in `cur`; once every wave holds its own,
+  // the stage takes tile it + S, and tile it + 1's are read behind the products.
+  auto body = [&](int it, Frags& cur, Frags& nxt) {
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 2) * kLoads) : "memory");
+    issue(it + S, stage);
+    stage = stage + 1 == S ? 0 : stage + 1;
+    read(stage, nxt);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(cur);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    bind(nxt);
+  };
+#pragma unroll 1
+  for (int it = 0; it < iters; it += 2) {
+    body(it, fa, fb);
+    if (it + 1 < iters) body(it + 1, fb, fa);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // no load lands in the rings any more
+  if constexpr (KG > 1) {
+    __syncthreads();
+    char* const sums = &lds[0][0];
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < TB; ++j)
+          *reinterpret_cast<f32x4_t*>(sums + ((((kg - 1) * 4 + wave) * NB * TB + i * TB + j) * 64 + lane) * 16) = acc[i][j];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int g = 0; g < KG - 1; ++g)
+#pragma unroll
+      for (int i = 0; i < NB; ++i)
+#pragma unroll
+        for (int j = 0; j < TB; ++j)
+          acc[i][j] += *reinterpret_cast<const f32x4_t*>(sums + (((g * 4 + wave) * NB * TB + i * TB + j) * 64 + lane) * 16);
+  }
+  const bool vec = ((reinterpret_cast<uintptr_t>(p.y) | (kEpi == 1 ? reinterpret_cast<uintptr_t>(p.res) : 0)) & 7u) == 0 &&
+                   p.ldy % 4 == 0;
+#pragma unroll
+  for (int j = 0; j < TB; ++j) {
+    const int t = t0 + 16 * (TB * wx + j) + fr;
+    if (t >= p.t) continue;
+#pragma unroll
+    for (int i = 0; i < (kEpi == 3 ? NB / 2 : NB); ++i) {
+      const int n = n0 + wrow(i) + 4 * fg;
+      if (n >= p.n) continue;
+      _Float16* dst = reinterpret_cast<_Float16*>(p.y) + (long long)t * p.ldy + n;
+      const _Float16* res = reinterpret_cast<const _Float16*>(p.res) + (long long)t * p.ldy + n;
+      f16x4_t v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        if constexpr (kEpi == 3) {
+          const float gh = (float)to_f16(acc[i][j][r]);
+          const float uh = (float)to_f16(acc[i + NB / 2][j][r]);
+          const float e = exp2_rep(-uh * kLog2e);
+          v[r] = to_f16(gh * (uh / (1.0f + e)));
+        } else {
+          v[r] = to_f16(acc[i][j][r]);
+        }
+      }
+      if (vec && n + 4 <= p.n) {
+        if constexpr (kEpi == 1) {
+          const f16x4_t rv = *reinterpret_cast<const f16x4_t*>(res);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = (_Float16)((float)rv[r] + (float)v[r]);
+        }
+        *reinterpret_cast<f16x4_t*>(dst) = v;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (n + r < p.n) dst[r] = kEpi == 1 ? (_Float16)((float)res[r] + (float)v[r]) : v[r];
+      }
+    }
+  }
+}
 
 // Large-M product on a ring of direct-to-LDS stages (M >= 128: the matrix-core
 // prefill's passes): a 128 x 128 workgroup tile computed as Y^T = W X^T, so
@@ -1224,10 +1544,11 @@ hipError_t launch_swiglu_batched(const uint16_t* g, const uint16_t* u, uint16_t*
   return hipGetLastError();
 }
 
-// Tile choice of a plain product from kRingMinRows tokens: 192 x 256 where
+// Tile choice of a product from kRingMinRows tokens: 192 x 256 where
 // that grid covers every CU (2048-token QKV: 256 tiles), else 128 x 128 where
 // that grid covers at least half of them (a 128 x 128 grid of 192 tiles ran
-// the 512-token QKV product as fast as hipBLASLt), else the 64 x 64 tile.
+// the 512-token QKV product as fast as hipBLASLt), else a short prompt's
+// (pick_short).
 enum class GemmTile { k64, k128, k192 };
 
 // The 128 x 128 tile's buffer loads take 32-bit byte offsets up to a tile past each operand's end.
@@ -1247,6 +1568,71 @@ static GemmTile pick_tile(const BatchedGemvParams& p, int rows_per_out) {
   if (big >= cus && offsets32) return GemmTile::k192;
   const long long mid = (long long)((p.n * rows_per_out + kRgN - 1) / kRgN) * ((p.t + kRgT - 1) / kRgT);
   return 2 * mid >= cus && ring128_offsets32(p) ? GemmTile::k128 : GemmTile::k64;
+}
+
+// Products that would take the 64 x 64 tile: the shape by the time of its rounds
+// of workgroups, `cus` at a time.  Measured per round and K tile of 64 (us; cold
+// weights, n = 2048-11008 rows, K = 2048 and 5504): 64 x 64 0.29, 32 x 32 and 32 x 16
+// with K shared out over eight waves 0.12 for one round and 0.157 each for more,
+// 32 x 64 0.24 and 64 x 128 0.50 in two K groups.  Between equals the smaller tile,
+// which has more of the device at work.
+enum class ShortTile { k64, kWave32x16, kWave32x32, kGroup32x64, kGroup64x128 };
+
+static ShortTile pick_short(const BatchedGemvParams& p, int rows_per_out) {
+  // lane offsets stay below 2^31 (rows of 128 tokens or 64 weights past a workgroup's base)
+  if (p.ldx >= (1LL << 23) || p.k >= (1 << 23)) return ShortTile::k64;
+  const long long cus = device_cus();
+  const long long rows = (long long)p.n * rows_per_out;
+  auto tiles = [&](int tn, int tt) { return (rows + tn - 1) / tn * ((p.t + tt - 1) / tt); };
+  if (tiles(32, 16) >= (1 << 20)) return ShortTile::k64;
+  auto rounds = [&](int tn, int tt) { return (tiles(tn, tt) + cus - 1) / cus; };
+  auto wave = [&](int tn, int tt) { return rounds(tn, tt) == 1 ? 120 : 157 * rounds(tn, tt); };
+  ShortTile best = ShortTile::kWave32x16;
+  long long cost = wave(32, 16);
+  auto take = [&](ShortTile t, long long c) {
+    if (c < cost) {
+      best = t;
+      cost = c;
+    }
+  };
+  take(ShortTile::kWave32x32, wave(32, 32));
+  if (rows_per_out == 1) take(ShortTile::kGroup32x64, 240 * rounds(32, 64));
+  take(ShortTile::k64, 290 * rounds(64, 64));
+  take(ShortTile::kGroup64x128, 500 * rounds(64, 128));
+  return best;
+}
+
+template <int NB, int TB, int W, int S, int kEpi>
+static void launch_wavek(const BatchedGemvParams& p, hipStream_t stream) {
+  constexpr int kOut = kEpi == 3 ? 8 * NB : 16 * NB;
+  const dim3 grid((unsigned)(((p.n + kOut - 1) / kOut) * ((p.t + 16 * TB - 1) / (16 * TB))));
+  hipLaunchKernelGGL((gemm_nt_wavek_kernel<NB, TB, W, S, kEpi>), grid, dim3(64 * W), 0, stream, p);
+}
+
+template <int NB, int TB, int WW, int KG, int S, int kEpi>
+static void launch_kgroup(const BatchedGemvParams& p, hipStream_t stream) {
+  constexpr int kN = 16 * NB * WW, kT = 16 * TB * (4 / WW), kOut = kEpi == 3 ? kN / 2 : kN;
+  const dim3 grid((unsigned)(((p.n + kOut - 1) / kOut) * ((p.t + kT - 1) / kT)));
+  hipLaunchKernelGGL((gemm_nt_kgroup_kernel<NB, TB, WW, KG, S, kEpi>), grid, dim3(256 * KG), 0, stream, p);
+}
+
+template <int kEpi>
+static hipError_t launch_short(const BatchedGemvParams& p, hipStream_t stream) {
+  switch (pick_short(p, kEpi == 3 ? 2 : 1)) {
+    case ShortTile::kWave32x16: launch_wavek<2, 1, 8, 3, kEpi>(p, stream); break;
+    case ShortTile::kWave32x32: launch_wavek<2, 2, 8, 2, kEpi>(p, stream); break;
+    case ShortTile::kGroup32x64:
+      if constexpr (kEpi != 3) launch_kgroup<2, 1, 1, 2, 6, kEpi>(p, stream);
+      break;
+    case ShortTile::kGroup64x128: launch_kgroup<2, 4, 2, 2, 3, kEpi>(p, stream); break;
+    case ShortTile::k64: {
+      constexpr int kOut = kEpi == 3 ? kMmTile / 2 : kMmTile;
+      hipLaunchKernelGGL(gemm_nt_mfma_kernel<kEpi>, dim3((p.n + kOut - 1) / kOut, (p.t + kMmTile - 1) / kMmTile),
+                         dim3(256), 0, stream, p);
+      break;
+    }
+  }
+  return hipGetLastError();
 }
 
 hipError_t launch_gemm_mfma(const BatchedGemvParams& p, int epi, hipStream_t stream) {
@@ -1269,14 +1655,8 @@ hipError_t launch_gemm_mfma(const BatchedGemvParams& p, int epi, hipStream_t str
       return hipGetLastError();
     }
     default:
-      break;
+      return epi == 0 ? launch_short<0>(p, stream) : launch_short<1>(p, stream);
   }
-  const dim3 grid((p.n + kMmTile - 1) / kMmTile, (p.t + kMmTile - 1) / kMmTile);
-  if (epi == 0)
-    hipLaunchKernelGGL(gemm_nt_mfma_kernel<0>, grid, dim3(256), 0, stream, p);
-  else
-    hipLaunchKernelGGL(gemm_nt_mfma_kernel<1>, grid, dim3(256), 0, stream, p);
-  return hipGetLastError();
 }
 
 hipError_t launch_gemm_mfma_swiglu(const BatchedGemvParams& p, hipStream_t stream) {
@@ -1292,34 +1672,25 @@ hipError_t launch_gemm_mfma_swiglu(const BatchedGemvParams& p, hipStream_t strea
                          dim3((unsigned)(((p.n + kRgN / 2 - 1) / (kRgN / 2)) * ((p.t + kRgT - 1) / kRgT))),
                          dim3(256), 0, stream, p);
       break;
-    default: {
-      const dim3 grid((p.n + kMmTile / 2 - 1) / (kMmTile / 2), (p.t + kMmTile - 1) / kMmTile);
-      hipLaunchKernelGGL(gemm_nt_mfma_kernel<3>, grid, dim3(256), 0, stream, p);
-      break;
-    }
+    default:
+      return launch_short<3>(p, stream);
   }
   return hipGetLastError();
 }
 
-// Splits K over up to kGemmMaxSplits slices of whole 64-wide tiles when the
-// product's grid leaves CUs idle and the workspace holds the slices' fp32
-// partials; one launch then adds the slices in order with the epilogue
-// (splitk_fold_kernel).  From kRingMinRows tokens with n a multiple of 4 the
-// slices run on the 128 x 128 ring tile (the 256-token c_proj product: 32
-// tiles of K = 5504), below it on the 64 x 64 tile.
+// Where the product takes 128 x 128 tiles and they fill at most half of the
+// device (1023 tokens of 2048 rows: 128 tiles), splits K over two slices of whole
+// 64-wide tiles when n is a multiple of 4 and the workspace holds the slices' fp32
+// partials; one launch then adds them in order with the epilogue
+// (splitk_fold_kernel): a 1023-token matrix-core prompt of 24 layers 5.13 ms
+// against 5.49 unsplit.  Fewer tokens share K out inside a workgroup
+// (launch_short), with no second launch: prompts of 127 / 255 / 511 / 800 tokens
+// 1.72 / 2.23 / 3.39 / 4.40 ms, split 2.02 / 2.66 / 3.85 / 5.01.
 hipError_t launch_gemm_mfma_split(const BatchedGemvParams& p, int epi, float* workspace,
                                   size_t workspace_bytes, hipStream_t stream) {
   if (p.k < 64 || p.k % 64 != 0 || p.t < 1 || p.n < 1) return hipErrorInvalidValue;
-  const GemmTile tile = pick_tile(p, 1);
-  const bool ring = p.t >= kRingMinRows && p.n % 4 == 0 && tile != GemmTile::k192 && ring128_offsets32(p) &&
-                    ((reinterpret_cast<uintptr_t>(p.y) | reinterpret_cast<uintptr_t>(p.res)) & 7u) == 0 &&
-                    p.ldy % 4 == 0;
-  const int tn = ring ? kRgN : kMmTile, tt = ring ? kRgT : kMmTile;
-  const long long tiles = (long long)((p.n + tn - 1) / tn) * ((p.t + tt - 1) / tt);
-  const int cus = device_cus();
-  int splits = 1;
-  if (workspace && tile != GemmTile::k192 && tiles < cus)
-    splits = (int)std::min<long long>(kGemmMaxSplits, (cus + tiles - 1) / tiles);
+  const long long tiles = (long long)((p.n + kRgN - 1) / kRgN) * ((p.t + kRgT - 1) / kRgT);
+  int splits = workspace && pick_tile(p, 1) == GemmTile::k128 && p.n % 4 == 0 && 2 * tiles <= device_cus() ? 2 : 1;
   if (splits > 1) {
     // slices of whole K tiles, none empty, as many as the workspace holds
     while (splits > 1 && (size_t)splits * p.t * p.n * sizeof(float) > workspace_bytes) --splits;
@@ -1329,12 +1700,7 @@ hipError_t launch_gemm_mfma_split(const BatchedGemvParams& p, int epi, float* wo
       BatchedGemvParams q = p;
       q.part = workspace;
       q.kslice = kslice;
-      if (ring)
-        hipLaunchKernelGGL(gemm_nt_ring128_kernel<2>, dim3((unsigned)tiles, splits), dim3(256), 0, stream, q);
-      else
-        hipLaunchKernelGGL(gemm_nt_mfma_kernel<2>,
-                           dim3((p.n + kMmTile - 1) / kMmTile, (p.t + kMmTile - 1) / kMmTile, splits),
-                           dim3(256), 0, stream, q);
+      hipLaunchKernelGGL(gemm_nt_ring128_kernel<2>, dim3((unsigned)tiles, splits), dim3(256), 0, stream, q);
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return e;
       const dim3 fgrid((unsigned)(((long long)p.t * p.n + 255) / 256));

@@ -171,6 +171,58 @@ def test_mfma_mode_within_fp32_summation_bound(qdiy, m, n, k, with_res):
     assert np.all(np.abs(got - want) <= tol), float(np.max(np.abs(got - want) - tol))
 
 
+@pytest.mark.parametrize("m,n,k", [
+    # 32 x 16 and 32 x 32 tiles, K over eight waves: fewer K tiles than waves, a wave
+    # with one more than another, ragged rows and tokens
+    (1, 32, 64), (16, 33, 64 * 7), (17, 31, 64 * 9), (33, 2050, 64 * 17), (100, 2048, 64 * 11),
+    # 32 x 64 tiles in two K groups: odd and even K tiles, one alone; ragged tokens
+    (63, 6144, 64), (49, 6112, 64 * 3), (64, 6100, 64 * 8),
+    # 64 x 64 and 64 x 128 tiles (two rounds and one of a device's workgroups)
+    (90, 6000, 64 * 5), (100, 11008, 64 * 3), (127, 11000, 64 * 2), (128, 10950, 64),
+    # from 128 tokens where the ring tiles would leave CUs idle
+    (200, 1024, 64 * 6), (140, 520, 64 * 13)])
+@pytest.mark.parametrize("form", ["plain", "residual", "swiglu"])
+def test_mfma_short_prompt_tiles(qdiy, m, n, k, form):
+    """The short-prompt shapes of both matrix-core products at their edges, with padded x
+    rows and y at an odd element offset (no 8-byte stores) when m is odd; nothing is
+    written outside y's rows.  Bounds as in the tests around this one."""
+    rng = np.random.default_rng(3 * m + n + k)
+    ldx, off, pad = k + 8, m % 2, 0 if m % 2 else 4
+    ldy = n + pad
+    if form == "swiglu":
+        n = max(1, n // 2)                              # two W rows per output: the same tiles
+        ldy = n + pad
+    x, W, W2 = normal_f16(rng, (m, ldx)), normal_f16(rng, (n, k), 0.02), normal_f16(rng, (n, k), 0.02)
+    R = normal_f16(rng, (m, ldy))
+    y = torch.full((off + m * ldy + 8,), 9.0, dtype=torch.float16, device="cuda")
+    if form == "swiglu":
+        qdiy.gemm_swiglu(_dev(x.reshape(-1)), _dev(W.reshape(-1)), _dev(W2.reshape(-1)), y[off:], m, n, k, ldx=ldx,
+                         ldy=ldy)
+    else:
+        qdiy.gemm_nt(_dev(x.reshape(-1)), _dev(W.reshape(-1)), y[off:], m, n, k, ldx=ldx, ldy=ldy,
+                     residual=_dev(R.reshape(-1)) if form == "residual" else None, mode=qdiy.GEMM_MFMA)
+    torch.cuda.synchronize()
+    out = y.cpu().numpy()
+    rows = out[off:off + m * ldy].reshape(m, ldy)
+    assert np.all(rows[:, n:] == 9.0) and np.all(out[:off] == 9.0) and np.all(out[off + m * ldy:] == 9.0)
+    got = rows[:, :n].astype(np.float64)
+    x64 = x[:, :k].astype(np.float64)
+    s, bs = x64 @ W.astype(np.float64).T, k * 2.0 ** -23 * (np.abs(x64) @ np.abs(W.astype(np.float64)).T)
+    if form == "plain":
+        want, tol = s, ulp16(s) + bs
+    elif form == "residual":
+        h = s.astype(np.float16).astype(np.float64)
+        want = R[:, :n].astype(np.float64) + h
+        tol = ulp16(want) + ulp16(h) + bs + ulp16(s)
+    else:
+        u, bu = x64 @ W2.astype(np.float64).T, k * 2.0 ** -23 * (np.abs(x64) @ np.abs(W2.astype(np.float64)).T)
+        g16, u16 = s.astype(np.float16).astype(np.float64), u.astype(np.float16).astype(np.float64)
+        silu = u16 / (1.0 + np.exp(-u16))
+        want = g16 * silu
+        tol = np.abs(silu) * (ulp16(g16) + bs) + np.abs(g16) * 1.1 * (ulp16(u16) + bu) + 2 * ulp16(want)
+    assert np.all(np.abs(got - want) <= tol), float(np.max(np.abs(got - want) - tol))
+
+
 @pytest.mark.parametrize("m,n,k,ldy", [(37, 100, 512, 100), (127, 1368, 2048, 1368),
                                         # from 128 rows: the 64 x 64 tile (n = 130, a strided
                                         # output), the 128 x 128 ring tile (a ragged last tile at
