@@ -569,8 +569,8 @@ __global__ __launch_bounds__(NW * 64) void decode_attention_scan_kernel(AttnPara
 // vector instructions, which share the same units, and half the time of a
 // workgroup's short life (16 rows per wave up to 1024 rows) is its first loads,
 // its folds and its end.  16 heads, whole calls: 256 queries from row 768 on
-// 171 -> 65 us (14 of it the merge kernel), from 2000 472 -> 105, from 5000
-// 1400 -> 263; 127 queries from row 0 16.6 -> 10 us.
+// 171 -> 59 us (7 of it the merge kernel), from 2000 472 -> 100, from 5000
+// 1400 -> 258; 127 queries from row 0 16.6 -> 10 us.
 //
 // A wave takes 16 rows at a time: one tile of 4-row groups (U = 4) or two
 // consecutive ones of 2-row groups.  NW is the plan's waves (the order of the
@@ -749,15 +749,16 @@ __device__ __forceinline__ void prefill_block(const AttnParams& p, PrefillLds<NW
 #pragma unroll
       for (int r = 0; r < 4; ++r) s[r] = row_at(blk, g, r) < n_q ? sum[r] * p.scale_log2 : -__builtin_inff();
     };
-    // One tile's softmax step: s becomes the weights; returns the rescale.
-    auto softmax = [&](int tl) {
+    // One tile's softmax step: s becomes the weights; returns the rescale (of an
+    // empty state, at the wave's first tile, there is nothing to rescale).
+    auto softmax = [&](int tl, bool start) {
       float mt = s[tl * U];
 #pragma unroll
       for (int u = 1; u < U; ++u) mt = fmaxf(mt, s[tl * U + u]);
       const float mn = fmaxf(m, mt);
       const float base = safe_base(mn);
-      const float alpha = exp2_rep_nonpos(m - base);
-      l *= alpha;
+      const float alpha = start ? 0.0f : exp2_rep_nonpos(m - base);
+      if (!start) l *= alpha;
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         s[tl * U + u] = exp2_rep_nonpos(s[tl * U + u] - base);
@@ -829,10 +830,10 @@ __device__ __forceinline__ void prefill_block(const AttnParams& p, PrefillLds<NW
     if (w != wave) load(blk);
     if constexpr (kOne) {
       scores(blk);
-      softmax(0);
+      softmax(0, true);
       const bool two = kTiles == 2 && blk + kStep < nmax;   // some query has the second tile
       if (two) {
-        const float alpha = softmax(kTiles - 1);
+        const float alpha = softmax(kTiles - 1, false);
         reinterpret_cast<float*>(&lds.alpha[w][ql])[g] = alpha;
       }
       meet();
@@ -852,7 +853,7 @@ __device__ __forceinline__ void prefill_block(const AttnParams& p, PrefillLds<NW
         for (int tl = 0; tl < kTiles; ++tl) {
           if (tl > 0 && blk + tl * kStep >= nmax) break;   // no query has this tile
           const float m0 = m;
-          const float alpha = softmax(tl);
+          const float alpha = softmax(tl, start && tl == 0);
           // as in the scan, the rescale changes no bit where no maximum rose
           if (!(start && tl == 0) && __builtin_amdgcn_ballot_w64(m != m0)) {
             reinterpret_cast<float*>(&lds.alpha[w][ql])[g] = alpha;
@@ -1067,6 +1068,57 @@ __global__ __launch_bounds__(kMergeThreads) void decode_attention_merge_kernel(A
     ov[j] = src.o4(cc);
   }
   merge_fold(ml, ov, splits, src, lds, out + h * kD);
+}
+
+// decode_attention_merge_kernel<true> for at most SMAX splits: a wave per (query,
+// head), lane l its dims 2 l and 2 l + 1, so nothing passes through LDS and no
+// barrier is waited at.  All partials are loaded at once; lane c forms split c's
+// weight; the sums are merge_fold's, slice by slice (split c in slice c % 8) and
+// then the slices in order.  What bounds it is reading the partials once: 34 MB for
+// 256 queries of 16 heads over 16 splits, 7.2 us (4.7 TB/s; 9.1 us with each load
+// moved to its use; 13.6 us as two launches of a workgroup per (query, head)).
+template <int SMAX>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(AttnParams p, int tokens) {
+  constexpr int P = kMergeSlices;
+  const int lane = threadIdx.x & 63;
+  const int i = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (i >= tokens * p.num_heads) return;                // whole wave
+  const int b = i / p.num_heads, h = i - b * p.num_heads;
+  int splits, rows, block;
+  auto_plan(p.seqlen + b, p.num_cus, p.num_heads, p.long_inter != 0, &splits, &rows, &block);
+  const long long first = ((long long)b * p.num_heads + h) * p.split_stride;
+  f32x2 o[SMAX];
+#pragma unroll
+  for (int c = 0; c < SMAX; ++c)
+    o[c] = *reinterpret_cast<const f32x2*>(p.part_o + (first + min(c, splits - 1)) * kD + 2 * lane);
+  const float2 ml = p.part_ml[first + min(lane, splits - 1)];
+  // every load before the first use (the compiler would move each into its branch below)
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int c = 0; c < SMAX; ++c) asm volatile("" : "+v"(o[c]));
+  const float M = wave64_max(ml.x);
+  const float w = exp2_rep_nonpos(ml.x - safe_base(M));
+  float L = 0.0f, o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+  for (int s = 0; s < P; ++s) {
+    float ll = 0.0f, a0 = 0.0f, a1 = 0.0f;
+#pragma unroll
+    for (int c = s; c < SMAX; c += P)
+      if (c < splits) {
+        const float wc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), c));
+        const float lc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ml.y), c));
+        ll = __builtin_fmaf(wc, lc, ll);
+        a0 = __builtin_fmaf(wc, o[c][0], a0);
+        a1 = __builtin_fmaf(wc, o[c][1], a1);
+      }
+    L = s == 0 ? ll : L + ll;
+    o0 = s == 0 ? a0 : o0 + a0;
+    o1 = s == 0 ? a1 : o1 + a1;
+  }
+  f16x2 out;
+  out[0] = to_f16(o0 / L);
+  out[1] = to_f16(o1 / L);
+  *reinterpret_cast<f16x2*>(p.out + b * p.out_batch_stride + h * kD + 2 * lane) = out;
 }
 
 // ---------------------------------------------------------------------------
@@ -1765,10 +1817,20 @@ hipError_t launch_decode_attention_split_batch(const AttnParams& p, int rows_per
     else
       hipLaunchKernelGGL((decode_attention_scan_kernel<4, 2, true, true>), scan_grid, dim3(256), 0, stream, p);
   }
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((decode_attention_merge_kernel<true>), dim3(p.num_heads, tokens),
-                     dim3(kMergeThreads), 0, stream, p);
+  return hipGetLastError();
+}
+
+hipError_t launch_decode_attention_merge_batch(const AttnParams& p, int tokens, hipStream_t stream) {
+  const dim3 grid((unsigned)((tokens * p.num_heads + 3) / 4));
+  if (p.split_stride <= 16)
+    hipLaunchKernelGGL(prefill_merge_kernel<16>, grid, dim3(256), 0, stream, p, tokens);
+  else if (p.split_stride <= 32)
+    hipLaunchKernelGGL(prefill_merge_kernel<32>, grid, dim3(256), 0, stream, p, tokens);
+  else if (p.split_stride <= 64)
+    hipLaunchKernelGGL(prefill_merge_kernel<64>, grid, dim3(256), 0, stream, p, tokens);
+  else
+    hipLaunchKernelGGL((decode_attention_merge_kernel<true>), dim3(p.num_heads, tokens),
+                       dim3(kMergeThreads), 0, stream, p);
   return hipGetLastError();
 }
 

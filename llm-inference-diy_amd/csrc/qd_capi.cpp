@@ -59,7 +59,7 @@ using qd::hip_fail;
 constexpr int kFusedMaxRows = 224;
 constexpr int kFusedMaxRowsX = 128;
 using qd::kXMergeMaxRows;
-constexpr int kPrefillBatch = 256;   // split-plan prefill queries per batched launch pair
+constexpr int kPrefillBatch = 256;   // split-plan prefill queries per merge
 
 qd::AttnPlan plan_fused(int seqlen) {
   qd::AttnPlan plan;
@@ -350,9 +350,9 @@ int attention_prefill(qd_ctx* ctx, const uint16_t* q, long long q_stride, const 
     const hipError_t e = qd::launch_decode_attention_fused_batch(p, n_fused, stream);
     if (e != hipSuccess) return hip_fail(e, "batched fused attention launch");
   }
-  // The others take split plans.  Runs of consecutive queries whose plans
-  // share a tile depth go out as one batched split launch pair, every query
-  // under its own plan (at most kPrefillBatch queries per pair).
+  // The others take split plans, at most kPrefillBatch queries at a time: runs
+  // of consecutive queries whose plans share a tile shape go out as one batched
+  // scan each, every query under its own plan, and one merge folds them all.
   if (n_fused >= tokens) return QD_OK;
   if (!ctx->pf_part_o) {
     // slots for kPrefillBatch queries x H heads x the largest automatic split count
@@ -369,28 +369,45 @@ int attention_prefill(qd_ctx* ctx, const uint16_t* q, long long q_stride, const 
     ctx->pf_tokens = kPrefillBatch;
     ctx->pf_stride = stride;
   }
-  for (int t = n_fused; t < tokens;) {
-    const qd::AttnPlan first = plan_auto(ctx, pos0 + t + 1);
-    // no wave of the plan's four has more than 16 rows
-    auto one_tile = [](const qd::AttnPlan& pl) { return !pl.block_rows && pl.rows_per_split <= 64; };
-    int t1 = t + 1, max_splits = first.splits;
-    for (; t1 < tokens && t1 - t < ctx->pf_tokens; ++t1) {
-      const qd::AttnPlan pl = plan_auto(ctx, pos0 + t1 + 1);
-      if (pl.rows_per_tile != first.rows_per_tile || one_tile(pl) != one_tile(first)) break;
-      max_splits = std::max(max_splits, pl.splits);
-    }
-    if (max_splits > ctx->pf_stride)
-      return fail(QD_EINVAL, "internal: %d splits above the prefill scratch's %d", max_splits, ctx->pf_stride);
-    qd::AttnParams p = make_params(ctx, q + t * q_stride, k, v, out + t * out_stride, pos0 + t + 1, first);
+  auto params = [&](int t) {                   // queries from t on, partials from slot 0 on
+    qd::AttnParams p = make_params(ctx, q + t * q_stride, k, v, out + t * out_stride, pos0 + t + 1,
+                                   plan_auto(ctx, pos0 + t + 1));
     p.q_batch_stride = q_stride;
     p.out_batch_stride = out_stride;
     p.part_o = ctx->pf_part_o;
     p.part_ml = ctx->pf_part_ml;
     p.num_cus = ctx->num_cus;
+    return p;
+  };
+  // no wave of the plan's four has more than 16 rows
+  auto one_tile = [](const qd::AttnPlan& pl) { return !pl.block_rows && pl.rows_per_split <= 64; };
+  for (int t0 = n_fused; t0 < tokens;) {
+    const int t2 = std::min(tokens, t0 + ctx->pf_tokens);
+    int max_splits = 1;
+    for (int t = t0; t < t2; ++t) max_splits = std::max(max_splits, plan_auto(ctx, pos0 + t + 1).splits);
+    if (max_splits > ctx->pf_stride)
+      return fail(QD_EINVAL, "internal: %d splits above the prefill scratch's %d", max_splits, ctx->pf_stride);
+    for (int t = t0; t < t2;) {
+      const qd::AttnPlan first = plan_auto(ctx, pos0 + t + 1);
+      int t1 = t + 1;
+      for (; t1 < t2; ++t1) {
+        const qd::AttnPlan pl = plan_auto(ctx, pos0 + t1 + 1);
+        if (pl.rows_per_tile != first.rows_per_tile || one_tile(pl) != one_tile(first)) break;
+      }
+      qd::AttnParams p = params(t);
+      const size_t slot = (size_t)(t - t0) * ctx->cfg.num_heads * max_splits;
+      p.part_o += slot * 128;
+      p.part_ml += slot;
+      p.split_stride = max_splits;
+      const hipError_t e = qd::launch_decode_attention_split_batch(p, first.rows_per_tile, one_tile(first), t1 - t, stream);
+      if (e != hipSuccess) return hip_fail(e, "batched split attention launch");
+      t = t1;
+    }
+    qd::AttnParams p = params(t0);
     p.split_stride = max_splits;
-    const hipError_t e = qd::launch_decode_attention_split_batch(p, first.rows_per_tile, one_tile(first), t1 - t, stream);
-    if (e != hipSuccess) return hip_fail(e, "batched split attention launch");
-    t = t1;
+    const hipError_t e = qd::launch_decode_attention_merge_batch(p, t2 - t0, stream);
+    if (e != hipSuccess) return hip_fail(e, "batched attention merge launch");
+    t0 = t2;
   }
   return QD_OK;
 }

@@ -357,12 +357,14 @@ inline int round_robin_period(const unsigned* xcc, int count) {
 hipError_t launch_decode_attention_fused_batch(const AttnParams& p, int tokens, hipStream_t stream);
 // Split attention of `tokens` queries at once, token b over p.seqlen + b rows,
 // each under its own auto_split plan (the plan qd_decode_attention picks for
-// that length): one scan launch of num_heads * p.split_stride workgroups per
-// token or, from a few tokens on, per 16 of them (those past a token's split
-// count exit at once) and one merge launch.  Every token's plan must have
-// rows_per_tile tile rows and, with one_tile, contiguous splits of at most 64 rows.
+// that length): the scan, with num_heads * p.split_stride workgroups per token
+// or, from a few tokens on, per 16 of them (those past a token's split count exit
+// at once).  Every token's plan must have rows_per_tile tile rows and, with
+// one_tile, contiguous splits of at most 64 rows.  The merge then folds the
+// partials of any run of tokens.
 hipError_t launch_decode_attention_split_batch(const AttnParams& p, int rows_per_tile, bool one_tile, int tokens,
                                                hipStream_t stream);
+hipError_t launch_decode_attention_merge_batch(const AttnParams& p, int tokens, hipStream_t stream);
 hipError_t launch_qkv_bias_rope_cache(const RopeParams& p, hipStream_t stream);
 hipError_t launch_qkv_front(const QkvFrontParams& p, hipStream_t stream);
 hipError_t launch_proj_residual(const ProjResidualParams& p, hipStream_t stream);
