@@ -115,7 +115,8 @@ int qd_gemm_swiglu(const uint16_t* x, long long ldx, const uint16_t* w1, const u
  * scatter_interleaved_kernel), reading Q and the cache in place.
  *   mode QD_GEMM_EXACT: every query with the arithmetic qd_decode_attention
  *     uses at its length, batched (one fused launch for the queries of up to
- *     224 rows, scan + merge pairs for the others): outputs are bit-identical
+ *     224 rows; one split launch per run of queries with one tile shape and
+ *     one merge per 256 queries for the others): outputs are bit-identical
  *     to decoding the prompt token by token.  The first call with queries
  *     beyond 224 rows allocates the context's prefill scratch.
  *   mode QD_GEMM_MFMA: one causal FlashAttention launch on the matrix cores

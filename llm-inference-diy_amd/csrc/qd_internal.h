@@ -420,8 +420,8 @@ namespace qd {
 // (query t over pos0 + t + 1 rows; q and out rows q_stride / out_stride
 // elements apart), each with the arithmetic of qd_decode_attention's own plan
 // for its length: the fused-plan queries in one batched launch, the split-plan
-// queries in batched scan + merge pairs, one per run of queries that share a
-// tile depth.
+// queries in one launch per run that shares a tile shape and one merge per batch
+// of 256.
 int attention_prefill(qd_ctx* ctx, const uint16_t* q, long long q_stride, const uint16_t* k,
                       const uint16_t* v, uint16_t* out, long long out_stride, int pos0, int tokens,
                       hipStream_t stream);
