@@ -53,6 +53,7 @@
 
 #include "qd_device.h"
 #include "qd_front_device.h"
+#include "qd_dispatch.h"
 #include "qd_internal.h"
 
 namespace qd {
@@ -582,7 +583,6 @@ __global__ __launch_bounds__(NW * 64) void decode_attention_scan_kernel(AttnPara
 // one holds an infinity or a NaN the block takes the scan's own steps.
 // kSplit: the split's partials, in the batched scan's slots; else (fused plans)
 // the outputs.
-constexpr int kPfQ = 16;                       // queries per workgroup
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 template <int NW>
@@ -1770,26 +1770,9 @@ static void launch_scan_inter(const AttnParams& p, int waves, int rows_per_tile,
     hipLaunchKernelGGL((decode_attention_scan_kernel<4, 4, true, false, D, true>), grid, dim3(256), 0, stream, p);
 }
 
-// Whether a batched launch over `tokens` queries of p.seqlen rows on has them
-// share their rows (prefill_exact_kernel) or scans for each alone.  The shared
-// form's time is that of a block of 16 however few they are.  Kernel times, alone
-// / shared: fused plans 6.6 / 9.6 us at 32 queries, 8.2 / 9.0 at 48, 16.6 / 10 at
-// 127.  Split plans (with the merge; H heads, L rows) cross where H L tokens is
-// 60-100 thousand: H 16, L 300: 10.1 / 13.4 us at 8 queries, 14.7 / 13.5 at 16;
-// L 1000: 9.8 / 10.1 at 5, 13.9 / 10.2 at 8; H 8, L 600: 10.4 / 11.8 at 10, 15.3 /
-// 13.8 at 16; and from 4000 rows up at 6 queries (27.5 / 27.4 us: one block's
-// waves read a split's rows in turn).
-static bool prefill_shares_rows(const AttnParams& p, int tokens, bool split) {
-  if (!split) return tokens >= 56;
-  return tokens >= 6 && (long long)p.num_heads * p.seqlen * tokens >= 90000;
-}
-static unsigned prefill_blocks(const AttnParams& p, int tokens) {   // blocks of 16 lengths the queries touch
-  return (unsigned)((p.seqlen - 1 + tokens - 1) / kPfQ - (p.seqlen - 1) / kPfQ + 1);
-}
-
 hipError_t launch_decode_attention_fused_batch(const AttnParams& p, int tokens, hipStream_t stream) {
-  if (prefill_shares_rows(p, tokens, false)) {
-    hipLaunchKernelGGL((prefill_exact_kernel<16, 8, 4, false, true>), dim3(p.num_heads, prefill_blocks(p, tokens)),
+  if (prefill_shares_fused(p.num_heads, p.seqlen, tokens, p.num_cus)) {
+    hipLaunchKernelGGL((prefill_exact_kernel<16, 8, 4, false, true>), dim3(p.num_heads, prefill_blocks(p.seqlen, tokens)),
                        dim3(8 * 64), 0, stream, p, tokens);
   } else {
     hipLaunchKernelGGL((decode_attention_scan_kernel<16, 4, false>), dim3(p.num_heads, tokens),
@@ -1800,8 +1783,8 @@ hipError_t launch_decode_attention_fused_batch(const AttnParams& p, int tokens, 
 
 hipError_t launch_decode_attention_split_batch(const AttnParams& p, int rows_per_tile, bool one_tile, int tokens,
                                                hipStream_t stream) {
-  if (prefill_shares_rows(p, tokens, true)) {
-    const dim3 grid(p.num_heads * p.split_stride, prefill_blocks(p, tokens));
+  if (prefill_shares_split(p.num_heads, p.seqlen, tokens, p.num_cus)) {
+    const dim3 grid(p.num_heads * p.split_stride, prefill_blocks(p.seqlen, tokens));
     if (rows_per_tile == 4 && one_tile)
       hipLaunchKernelGGL((prefill_exact_kernel<4, 4, 4, true, true>), grid, dim3(256), 0, stream, p, tokens);
     else if (rows_per_tile == 4)

@@ -1,0 +1,59 @@
+"""The rules that choose a kernel from a call's sizes (csrc/qd_dispatch.h), compiled for
+the host: at sizes measured on both sides, on 256 compute units, the faster one."""
+import ctypes
+import os
+import subprocess
+
+import pytest
+
+from conftest import ROOT
+
+CUS = 256
+SHIM = r"""
+#include "qd_dispatch.h"
+extern "C" {
+int shares_fused(int heads, int seqlen, int tokens, int cus) { return qd::prefill_shares_fused(heads, seqlen, tokens, cus); }
+int shares_split(int heads, int seqlen, int tokens, int cus) { return qd::prefill_shares_split(heads, seqlen, tokens, cus); }
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    tmp = tmp_path_factory.mktemp("rules")
+    src, lib = tmp / "shim.cpp", tmp / "shim.so"
+    src.write_text(SHIM)
+    csrc = os.path.join(ROOT, "llm-inference-diy_amd", "csrc")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-I", csrc, "-o", str(lib), str(src)],
+                   check=True)
+    return ctypes.CDLL(str(lib))
+
+
+@pytest.mark.parametrize("heads,pos0,tokens,scan_us,shared_us", [
+    (1, 0, 56, 3.89, 7.35), (1, 0, 224, 4.91, 12.85), (2, 164, 60, 4.80, 12.89), (4, 0, 56, 4.07, 7.61),
+    (4, 0, 128, 5.97, 9.17), (4, 0, 224, 10.44, 12.87), (4, 124, 100, 7.09, 12.90), (8, 0, 56, 5.63, 7.65),
+    (8, 0, 96, 7.51, 9.08), (8, 0, 128, 9.34, 9.21), (8, 68, 60, 6.14, 9.22), (12, 0, 64, 7.39, 7.80),
+    (12, 0, 96, 10.67, 9.11), (12, 164, 60, 9.80, 12.96), (12, 124, 100, 13.91, 12.95), (16, 0, 48, 7.31, 7.56),
+    (16, 0, 56, 8.81, 7.72), (16, 0, 128, 16.34, 9.31), (20, 0, 56, 10.24, 7.78), (20, 194, 30, 9.85, 12.97),
+    (24, 0, 40, 8.79, 7.51), (32, 0, 20, 7.03, 7.11), (32, 0, 32, 8.78, 7.34), (32, 64, 16, 6.09, 8.88),
+    (64, 0, 24, 11.77, 7.36), (64, 64, 8, 6.02, 8.85), (64, 0, 128, 56.27, 16.18)])
+def test_fused_prompt_attention_takes_the_faster_form(rules, heads, pos0, tokens, scan_us, shared_us):
+    assert bool(rules.shares_fused(heads, pos0 + 1, tokens, CUS)) == (shared_us < scan_us)
+
+
+@pytest.mark.parametrize("heads,pos0,tokens,scan_us,shared_us", [
+    (1, 1000, 48, 11.9, 13.7), (1, 4000, 48, 35.9, 27.9), (4, 300, 64, 14.78, 15.76), (4, 1000, 12, 10.73, 11.98),
+    (4, 1000, 24, 15.50, 12.44), (4, 4000, 8, 12.86, 10.03), (8, 1000, 6, 8.1, 9.1), (8, 1000, 12, 10.6, 10.5),
+    (8, 2000, 6, 8.87, 9.37), (12, 600, 32, 19.3, 13.5), (16, 128, 64, 24.86, 20.46), (16, 300, 8, 8.51, 10.20),
+    (16, 1000, 4, 7.69, 9.24), (16, 1000, 6, 8.76, 9.24), (16, 1000, 8, 9.83, 9.32), (16, 2000, 6, 14.54, 13.38),
+    (16, 8000, 6, 54.63, 39.65), (20, 1000, 6, 11.50, 12.66), (20, 1000, 12, 17.1, 16.1), (24, 1000, 6, 12.26, 13.44),
+    (32, 600, 6, 10.43, 12.53), (32, 1000, 12, 22.7, 16.7), (64, 300, 6, 11.06, 14.76), (64, 300, 8, 12.27, 14.82),
+    (64, 1000, 8, 35.7, 19.6), (128, 128, 16, 20.15, 24.10), (128, 1000, 8, 76.6, 30.4)])
+def test_split_prompt_attention_takes_the_faster_form(rules, heads, pos0, tokens, scan_us, shared_us):
+    assert bool(rules.shares_split(heads, pos0 + 1, tokens, CUS)) == (shared_us < scan_us)
+
+
+def test_up_to_five_queries_of_split_plans_are_scanned(rules):
+    for heads in (1, 4, 16, 256, 4096):
+        for tokens in (1, 2, 5):
+            assert not rules.shares_split(heads, 100000, tokens, CUS)

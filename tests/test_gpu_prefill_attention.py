@@ -178,6 +178,21 @@ def test_exact_mode_shared_rows(qdiy, H, pos0, T, layout, bad_v):
         pr.close()
 
 
+@pytest.mark.parametrize("H,pos0,T,layout", [
+    # fused plans: the last count that is scanned and the first that is shared, with up
+    # to 128 and (heads the in-kernel merge leaves out) up to 224 rows
+    (8, 0, 96, "engine"), (8, 10, 118, "head_major"), (4, 0, 128, "engine"), (12, 124, 100, "engine"),
+    (12, 160, 64, "head_major"),
+    # split plans: 7 and 8 queries, across a block's edge, and more than 64 heads, whose plans
+    # change inside a block
+    (20, 1000, 7, "engine"), (20, 1000, 8, "engine"), (64, 300, 8, "engine"), (64, 290, 26, "engine"),
+    (96, 250, 20, "engine")])
+@pytest.mark.parametrize("bad_v", [False, True])
+def test_exact_mode_on_both_sides_of_the_sharing_rule(qdiy, H, pos0, T, layout, bad_v):
+    """Where the choice between the shared form and the scan lies: the same bits."""
+    test_exact_mode_shared_rows(qdiy, H, pos0, T, layout, bad_v)
+
+
 @pytest.mark.parametrize("H,pos0,T,layout,q_pad,out_pad",
                          CASES + [(16, 1792, 256, "engine", 4096, 0), (4, 0, 2048, "engine", 1024, 0),
                                   (16, 0, 2048, "engine", 4096, 0),      # a full pass at Qwen-1.8B's heads
