@@ -1070,15 +1070,16 @@ __global__ __launch_bounds__(kMergeThreads) void decode_attention_merge_kernel(A
   merge_fold(ml, ov, splits, src, lds, out + h * kD);
 }
 
-// decode_attention_merge_kernel<true> for at most SMAX splits: a wave per (query,
-// head), lane l its dims 2 l and 2 l + 1, so nothing passes through LDS and no
-// barrier is waited at.  All partials are loaded at once; lane c forms split c's
-// weight; the sums are merge_fold's, slice by slice (split c in slice c % 8) and
-// then the slices in order.  What bounds it is reading the partials once: 34 MB for
-// 256 queries of 16 heads over 16 splits, 7.2 us (4.7 TB/s; 9.1 us with each load
-// moved to its use; 13.6 us as two launches of a workgroup per (query, head)).
-template <int SMAX>
+// decode_attention_merge_kernel<true> for many queries of at most kWaveMergeSplits
+// splits: a wave per (query, head), lane l its dims 2 l and 2 l + 1, so nothing passes
+// through LDS and no barrier is waited at.  All partials are loaded at once; lane c
+// forms split c's weight; the sums are merge_fold's, slice by slice (split c in slice
+// c % 8) and then the slices in order.  What bounds it is reading the partials once:
+// 34 MB for 256 queries of 16 heads over 16 splits, 7.2 us (4.7 TB/s; 9.1 us with each
+// load moved to its use).  With little to read the wave's serial sums show instead:
+// prefill_merges_by_wave.
 __global__ __launch_bounds__(256) void prefill_merge_kernel(AttnParams p, int tokens) {
+  constexpr int SMAX = kWaveMergeSplits;
   constexpr int P = kMergeSlices;
   const int lane = threadIdx.x & 63;
   const int i = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1804,13 +1805,9 @@ hipError_t launch_decode_attention_split_batch(const AttnParams& p, int rows_per
 }
 
 hipError_t launch_decode_attention_merge_batch(const AttnParams& p, int tokens, hipStream_t stream) {
-  const dim3 grid((unsigned)((tokens * p.num_heads + 3) / 4));
-  if (p.split_stride <= 16)
-    hipLaunchKernelGGL(prefill_merge_kernel<16>, grid, dim3(256), 0, stream, p, tokens);
-  else if (p.split_stride <= 32)
-    hipLaunchKernelGGL(prefill_merge_kernel<32>, grid, dim3(256), 0, stream, p, tokens);
-  else if (p.split_stride <= 64)
-    hipLaunchKernelGGL(prefill_merge_kernel<64>, grid, dim3(256), 0, stream, p, tokens);
+  if (prefill_merges_by_wave(p.num_heads, tokens, p.split_stride))
+    hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((tokens * p.num_heads + 3) / 4)), dim3(256), 0, stream, p,
+                       tokens);
   else
     hipLaunchKernelGGL((decode_attention_merge_kernel<true>), dim3(p.num_heads, tokens),
                        dim3(kMergeThreads), 0, stream, p);

@@ -50,4 +50,19 @@ inline bool prefill_shares_split(int heads, int seqlen, int tokens, int cus) {
   return (long long)heads * seqlen * tokens >= need;
 }
 
+// Whether the partials of `tokens` queries are folded by a wave per (query, head)
+// (prefill_merge_kernel) or by a workgroup (decode_attention_merge_kernel).  The wave
+// adds its splits one after another, so it needs enough waves to read for all of them;
+// the workgroup has each slice's sums in its own threads and is the faster one until
+// the workgroups queue.  Whole calls, workgroup / wave us: 16 splits (16 heads) 1 query
+// after 1000 rows 6.2 / 6.5, 64 queries 32.8 / 34.8, 128 52.0 / 53.6, 256 89.7 / 88.4;
+// 8 splits (32 heads, 300 rows) 16 queries 11.9 / 12.1, 128 37.6 / 35.6, 256 80.7 / 74.5;
+// 4 splits (64 heads, 600 rows) 32 queries 31.6 / 29.7.  Over 17 and more splits the
+// wave's registers for all loads cost more than they gain: 32 splits (8 heads) 1 query
+// after 1000 rows 6.0 / 7.2; 64 (4 heads) 6.3 / 8.7, 256 queries 48.5 / 52.3.
+constexpr int kWaveMergeSplits = 16;
+inline bool prefill_merges_by_wave(int heads, int tokens, int splits) {
+  return splits <= kWaveMergeSplits && (long long)heads * tokens >= 192LL * splits;
+}
+
 }  // namespace qd

@@ -14,6 +14,7 @@ SHIM = r"""
 extern "C" {
 int shares_fused(int heads, int seqlen, int tokens, int cus) { return qd::prefill_shares_fused(heads, seqlen, tokens, cus); }
 int shares_split(int heads, int seqlen, int tokens, int cus) { return qd::prefill_shares_split(heads, seqlen, tokens, cus); }
+int merges_by_wave(int heads, int tokens, int splits) { return qd::prefill_merges_by_wave(heads, tokens, splits); }
 }
 """
 
@@ -57,3 +58,12 @@ def test_up_to_five_queries_of_split_plans_are_scanned(rules):
     for heads in (1, 4, 16, 256, 4096):
         for tokens in (1, 2, 5):
             assert not rules.shares_split(heads, 100000, tokens, CUS)
+
+
+@pytest.mark.parametrize("heads,tokens,splits,group_us,wave_us", [
+    (1, 1, 63, 6.14, 7.44), (4, 1, 64, 6.30, 8.73), (4, 64, 64, 20.31, 23.84), (4, 256, 64, 48.50, 52.32),
+    (8, 1, 32, 6.00, 7.23), (8, 128, 32, 31.06, 34.97), (12, 6, 21, 10.3, 11.3), (16, 1, 16, 6.16, 6.52),
+    (16, 16, 16, 11.31, 12.25), (16, 64, 16, 32.82, 34.76), (16, 128, 16, 52.02, 53.56), (16, 256, 16, 89.70, 88.43),
+    (20, 256, 12, 91.1, 86.6), (32, 256, 8, 80.7, 74.5), (64, 32, 4, 31.6, 29.7), (128, 48, 2, 82.7, 73.2)])
+def test_prompt_merge_takes_the_faster_form(rules, heads, tokens, splits, group_us, wave_us):
+    assert bool(rules.merges_by_wave(heads, tokens, splits)) == (wave_us < group_us)

@@ -193,6 +193,18 @@ def test_exact_mode_on_both_sides_of_the_sharing_rule(qdiy, H, pos0, T, layout, 
     test_exact_mode_shared_rows(qdiy, H, pos0, T, layout, bad_v)
 
 
+@pytest.mark.parametrize("H,pos0,T", [
+    # 16 splits: the last count whose partials a workgroup folds and the first that a wave does
+    (16, 700, 191), (16, 700, 192),
+    # fewer splits, down to two; query counts that leave waves of the last workgroup idle
+    (24, 300, 128), (20, 830, 117), (64, 280, 17), (96, 300, 9), (128, 200, 7),
+    # 1 to 3 heads, more than 64 splits: rows shared by 16 queries, and scanned
+    (1, 2000, 64), (2, 2000, 40), (3, 3000, 20), (1, 1500, 4), (3, 1500, 5), (2, 5000, 3)])
+def test_exact_mode_merge_forms(qdiy, H, pos0, T):
+    """Both merges of batched queries' partials at the edges of their ranges."""
+    test_exact_mode_shared_rows(qdiy, H, pos0, T, "engine", False)
+
+
 @pytest.mark.parametrize("H,pos0,T,layout,q_pad,out_pad",
                          CASES + [(16, 1792, 256, "engine", 4096, 0), (4, 0, 2048, "engine", 1024, 0),
                                   (16, 0, 2048, "engine", 4096, 0),      # a full pass at Qwen-1.8B's heads
