@@ -65,4 +65,19 @@ inline bool prefill_merges_by_wave(int heads, int tokens, int splits) {
   return splits <= kWaveMergeSplits && (long long)heads * tokens >= 192LL * splits;
 }
 
+// Whether an exact product of `tokens` rows with n weight rows of K goes to the two-row
+// FMA kernel (gemv_batched_kernel), which reads each weight row once and little else, or
+// to the fp32 matrix instructions.  Up to 4 tokens the first: two-row / matrix us at 4 /
+// 6 / 16 tokens, cold weights, 9.1 / 10.1 / 16.0 against 10.3 / 10.3 / 10.4 (6144 x
+// 2048), 5.8 / 6.5 / 10.4 against 6.1 / 6.0 / 6.2 (2048 x 2048), 10.6 / 12.7 / 22.0
+// against 11.3 / 11.2 / 11.4 (2048 x 5504).  From K = 7169 its workgroups have four waves,
+// no prefetch and a CU to themselves, so it stays the faster one only while they all run
+// at once: 1 / 4 tokens, K = 7176, 1024 rows 8.2 / 11.9 against 13.0 / 12.9, 2048 rows
+// 9.7 / 13.4 against 14.3 / 14.1, 4096 rows 17.7 / 24.6 against 17.1 / 15.6.
+constexpr int kWideTwoRowWg = 8;   // weight rows per workgroup of the two-row kernel from K = 7169
+inline bool exact_two_rows(int tokens, int n, int k, int cus) {
+  if (tokens > 4) return false;
+  return k <= 7168 || (n + kWideTwoRowWg - 1) / kWideTwoRowWg <= cus;
+}
+
 }  // namespace qd

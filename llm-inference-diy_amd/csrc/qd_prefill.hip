@@ -18,7 +18,7 @@
 //   rmsnorm_batched_kernel     T waves: xn[t] = RMSNorm(x[t]) * w
 //   gemm_exact_mfma_kernel     Y[t][n] = sum_k X[t][k] W[n][k], with an epilogue
 //                              (store as half, or residual add into the stream)
-//   gemv_batched_kernel        the same for up to 4 tokens: each weight row is
+//   gemv_batched_kernel        the same for up to 4 tokens (exact_two_rows): each weight row is
 //                              read once and kept in registers
 //   rope_batched_kernel        bias + RoPE + KV append per token (qd_rope_cache)
 //   swiglu_batched_kernel      act = half(g * (u / (1 + exp(-u))))
@@ -27,6 +27,7 @@
 #include <atomic>
 
 #include "qd_device.h"
+#include "qd_dispatch.h"
 #include "qd_internal.h"
 
 namespace qd {
@@ -46,6 +47,7 @@ constexpr int tok_tile(int nj) { return nj <= 8 ? 8 : (64 / nj) & ~1; }
 // wave may also use the accumulation registers): no scratch.  Which workgroup
 // computes a row does not change its sums.
 constexpr int gemv_waves(int nj) { return nj >= 15 ? 4 : 8; }
+static_assert(2 * gemv_waves(16) == kWideTwoRowWg, "the dispatch rule's rows per workgroup");
 
 // One wave per token: the same normalisation as the decode kernels' normalise()
 // (qd_decode_ops.hip), written out as fp16.
@@ -1480,20 +1482,14 @@ static int device_cus() {
   return v;
 }
 
-// From 5 tokens on the fp32 matrix instructions (qd_exact_gemm.hip; the same
-// bits), up to 4 tokens on the two-row FMA kernel, which reads each weight row
-// once and little else: kernel times at 4 / 6 / 16 tokens, cold weights, 9.1 /
-// 10.1 / 16.0 us against 10.3 / 10.3 / 10.4 (6144 x 2048), 5.8 / 6.5 / 10.4
-// against 6.1 / 6.0 / 6.2 (2048 x 2048), 10.6 / 12.7 / 22.0 against 11.3 / 11.2
-// / 11.4 (2048 x 5504).  From K = 7169 the two-row kernel's workgroups have four
-// waves and no prefetch and lose from one token (4096 x 8192: 20.5 against 16.8
-// us).  It also takes what the other kernel's 32-bit lane offsets or its
-// one-dimensional grid cannot.
+// On the fp32 matrix instructions (qd_exact_gemm.hip) or, for a few tokens
+// (exact_two_rows), on the two-row FMA kernel: the same bits.  That one also takes what
+// the other kernel's 32-bit lane offsets or its one-dimensional grid cannot.
 hipError_t launch_gemv_batched(const BatchedGemvParams& p, int epi, hipStream_t stream) {
   const int nj = (p.k + 511) / 512;
   if (nj < 1 || nj > 16) return hipErrorInvalidValue;
   const bool fits = p.ldx < (1LL << 26) && ((long long)p.n + 31) / 32 * (((long long)p.t + 31) / 32) < (1LL << 20);
-  if ((p.t > 4 || nj >= 15) && fits) return launch_gemm_exact_mfma(p, epi, device_cus(), stream);
+  if (fits && !exact_two_rows(p.t, p.n, p.k, device_cus())) return launch_gemm_exact_mfma(p, epi, device_cus(), stream);
   const int waves = gemv_waves(nj);
   const dim3 grid((p.n + 2 * waves - 1) / (2 * waves), (p.t + kTokPerWg - 1) / kTokPerWg);
   const size_t lds = (size_t)tok_tile(nj) * nj * 512 * sizeof(uint16_t);

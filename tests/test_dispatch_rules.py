@@ -15,6 +15,7 @@ extern "C" {
 int shares_fused(int heads, int seqlen, int tokens, int cus) { return qd::prefill_shares_fused(heads, seqlen, tokens, cus); }
 int shares_split(int heads, int seqlen, int tokens, int cus) { return qd::prefill_shares_split(heads, seqlen, tokens, cus); }
 int merges_by_wave(int heads, int tokens, int splits) { return qd::prefill_merges_by_wave(heads, tokens, splits); }
+int exact_two_rows(int tokens, int n, int k, int cus) { return qd::exact_two_rows(tokens, n, k, cus); }
 }
 """
 
@@ -67,3 +68,12 @@ def test_up_to_five_queries_of_split_plans_are_scanned(rules):
     (20, 256, 12, 91.1, 86.6), (32, 256, 8, 80.7, 74.5), (64, 32, 4, 31.6, 29.7), (128, 48, 2, 82.7, 73.2)])
 def test_prompt_merge_takes_the_faster_form(rules, heads, tokens, splits, group_us, wave_us):
     assert bool(rules.merges_by_wave(heads, tokens, splits)) == (wave_us < group_us)
+
+
+@pytest.mark.parametrize("tokens,n,k,two_rows_us,matrix_us", [
+    (1, 16, 8192, 6.55, 13.40), (4, 16, 8192, 11.34, 13.33), (1, 1024, 7176, 8.15, 13.03), (4, 2048, 7176, 13.36, 14.14),
+    (1, 2048, 8192, 11.32, 15.79), (2, 2048, 7680, 10.49, 14.86), (1, 4096, 8192, 20.42, 17.64),
+    (4, 4096, 7176, 24.55, 15.59), (5, 4096, 8192, 36.91, 16.91), (5, 2048, 7176, 16.19, 14.21), (4, 6144, 2048, 9.1, 10.3),
+    (4, 2048, 5504, 10.6, 11.3), (6, 2048, 5504, 12.7, 11.2), (16, 2048, 2048, 10.4, 6.2)])
+def test_exact_product_takes_the_faster_kernel(rules, tokens, n, k, two_rows_us, matrix_us):
+    assert bool(rules.exact_two_rows(tokens, n, k, CUS)) == (two_rows_us < matrix_us)

@@ -193,11 +193,10 @@ def test_prefill_batches_equal_token_by_token(qdiy):
 @pytest.mark.parametrize("hidden,inter", [(2560, 2600), (3584, 4104), (4096, 5120), (512, 5640),
                                           (1024, 8192)])
 def test_prefill_gemm_widths(qdiy, hidden, inter):
-    """The batched prefill GEMM at every row width the engine accepts: K = hidden
-    takes 5, 7 or 8 chunks of 512 per lane, K = inter 6-10 (with a ragged last
-    chunk, next-tile prefetch) and 12 or 16 (no prefetch: the registers are not
-    there).  41 prompt tokens span two 32-token groups and partial token tiles.
-    Greedy tokens and the last logits equal the oracle's bit for bit."""
+    """The batched prefill products at the widths of row the engine accepts: K = hidden of
+    5, 7 or 8 steps of 512, K = inter of 6-10 (with a ragged last step), 12 and 16.  41
+    prompt tokens fill two 16-token tiles and part of a third.  Greedy tokens and the last
+    logits equal the oracle's bit for bit."""
     cfg = qdiy.model_cfg(vocab_size=300, hidden_size=hidden, num_layers=1, num_heads=hidden // 128,
                          intermediate_size=inter, max_seqlen=48)
     img = qdiy.random_model_image(cfg, 31 + hidden + inter, 0.03, nthreads=8)

@@ -43,12 +43,11 @@ def _dev(a):
                                    (45, 4104, 1544), (300, 4100, 2000)])
 @pytest.mark.parametrize("with_res", [False, True])
 def test_exact_mode_is_the_decode_gemv(qdiy, m, n, k, with_res):
-    """Exact-mode rows against the oracle's decode GEMV, bit for bit.  From K = 1544 to
-    2048 with n >= 4096 the four-rows-per-wave kernel runs: (45, 4104, 1544) has a last
-    chunk of one lane, rows past n clamped in the last workgroup and odd token tiles;
-    (300, 4100, 2000) more than 256 tokens.  (256, 2048, 5504) runs 64 tokens per
-    workgroup in 4-token tiles.  The rows checked straddle the token tiles and the 32-
-    and 64-token workgroups."""
+    """Exact-mode rows against the oracle's decode GEMV, bit for bit: one token on the
+    two-row kernel, the others on the fp32 matrix instructions.  (45, 4104, 1544) has a
+    last chunk of K of one lane and a ragged last tile in both directions; (300, 4100,
+    2000) more than 256 tokens; (256, 2048, 5504) the widest K of the 1.8B shape.  The
+    rows checked straddle the 16- and 32-token tiles."""
     rng = np.random.default_rng(m * 1000 + n + k + with_res)
     x, W, R = normal_f16(rng, (m, k)), normal_f16(rng, (n, k), 0.02), normal_f16(rng, (m, n))
     y = torch.zeros(m * n, dtype=torch.float16, device="cuda")
@@ -123,6 +122,65 @@ def test_exact_mode_far_apart_rows(qdiy):
     take the two-row kernel: the same bits."""
     m, n, k, ldx = 6, 64, 264, 1 << 26
     rng = np.random.default_rng(6)
+    x, W = normal_f16(rng, (m, k)), normal_f16(rng, (n, k), 0.02)
+    far = torch.empty((m - 1) * ldx + k, dtype=torch.float16, device="cuda")
+    for i in range(m):
+        far[i * ldx:i * ldx + k] = _dev(x[i])
+    y = torch.zeros(m * n, dtype=torch.float16, device="cuda")
+    qdiy.gemm_nt(far, _dev(W.reshape(-1)), y, m, n, k, ldx=ldx, mode=qdiy.GEMM_EXACT)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().reshape(m, n)
+    for i in range(m):
+        assert _same(got[i], oracle.gemv(x[i], W.reshape(-1), n, k, 0, oracle.ORDER_WAVE64)), f"row {i}"
+
+
+@pytest.mark.parametrize("k", [1544, 2048, 4104, 5504, 6152, 7168, 7176, 8192])
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+@pytest.mark.parametrize("with_res", [False, True])
+def test_exact_mode_two_row_kernel(qdiy, m, k, with_res):
+    """Up to 4 tokens, every output bit for bit: the two-row kernel with 4 to 16 chunks of K
+    per lane, whole and ragged, with its next tile's loads in flight (up to 11 chunks) and
+    without, eight and (from K = 7169) four waves per workgroup; odd and even tokens, an odd
+    last row, padded x and y rows."""
+    n, ldx, pad = 37, k + 8, 3
+    rng = np.random.default_rng(17 * m + k + with_res)
+    x, W, R = normal_f16(rng, (m, ldx)), normal_f16(rng, (n, k), 0.02), normal_f16(rng, (m, n + pad))
+    y = torch.full((m * (n + pad) + 8,), 9.0, dtype=torch.float16, device="cuda")
+    qdiy.gemm_nt(_dev(x.reshape(-1)), _dev(W.reshape(-1)), y, m, n, k, ldx=ldx, ldy=n + pad,
+                 residual=_dev(R.reshape(-1)) if with_res else None, mode=qdiy.GEMM_EXACT)
+    torch.cuda.synchronize()
+    out = y.cpu().numpy()
+    got = out[:m * (n + pad)].reshape(m, n + pad)
+    assert np.all(got[:, n:] == 9.0) and np.all(out[m * (n + pad):] == 9.0)
+    for i in range(m):
+        if with_res:
+            want = oracle.proj_residual(x[i, :k], W.reshape(-1), R[i, :n], n, k)
+        else:
+            want = oracle.gemv(x[i, :k], W.reshape(-1), n, k, 0, oracle.ORDER_WAVE64)
+        assert _same(got[i, :n], want), f"row {i}"
+
+
+@pytest.mark.parametrize("n", [2048, 2049])
+def test_exact_mode_wide_rows_change_kernel(qdiy, n):
+    """K > 7168: up to 2048 weight rows on the two-row kernel, more on the matrix
+    instructions (256 compute units): the same bits."""
+    m, k = 2, 7176
+    rng = np.random.default_rng(n)
+    x, W = normal_f16(rng, (m, k)), normal_f16(rng, (n, k), 0.02)
+    y = torch.zeros(m * n, dtype=torch.float16, device="cuda")
+    qdiy.gemm_nt(_dev(x.reshape(-1)), _dev(W.reshape(-1)), y, m, n, k, mode=qdiy.GEMM_EXACT)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy().reshape(m, n)
+    for i in range(m):
+        assert _same(got[i], oracle.gemv(x[i], W.reshape(-1), n, k, 0, oracle.ORDER_WAVE64)), f"row {i}"
+
+
+@pytest.mark.parametrize("m,k", [(41, 264), (34, 2048), (37, 6152), (35, 8192)])
+def test_exact_mode_far_apart_rows_past_a_token_block(qdiy, m, k):
+    """More than 32 token rows 2^26 elements apart: the two-row kernel's second block of
+    tokens and its later tiles, with and without its prefetch."""
+    n, ldx = 24, 1 << 26
+    rng = np.random.default_rng(m + k)
     x, W = normal_f16(rng, (m, k)), normal_f16(rng, (n, k), 0.02)
     far = torch.empty((m - 1) * ldx + k, dtype=torch.float16, device="cuda")
     for i in range(m):
