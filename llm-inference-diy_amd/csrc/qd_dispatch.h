@@ -80,4 +80,43 @@ inline bool exact_two_rows(int tokens, int n, int k, int cus) {
   return k <= 7168 || (n + kWideTwoRowWg - 1) / kWideTwoRowWg <= cus;
 }
 
+// The matrix-core tile of a product that takes neither ring tile, over `rows` weight
+// rows (both weights' in the gate/up form, `paired`) and `tokens` of K: the one whose
+// rounds of workgroups, one per CU, cost least.  A round costs a start and an end,
+// whatever K, and a time per K tile of 64 (us, fitted to 1600 products of 16-40000 rows,
+// 1-400 tokens and K = 64-5504, cold weights, every tile timed on each):
+//   64 x 64                              1.7 + 0.33 per K tile
+//   32 x 32 and 32 x 16, K over eight waves  1.9 + 0.10 in a single round, 0.16 in more
+//   32 x 64, K over two groups           1.9 + 0.23
+//   64 x 128, K over two groups          1.9 + 0.42
+// With a residual the 64-row tiles end later the more tokens they hold, as each lane
+// reads it row by row: 0.03 us per token of 32, and 0.014 of 64 (20000 x 512, 32 tokens
+// 9.7 us without, 14.6 with; on 32 x 32 tiles 10.6 and 11.0).  The tiles so chosen are
+// 0.15% (with a residual 0.6%) slower than the best of the five on average; by the times
+// per K tile alone they were 1.3% and up to 71% (the start decides where K is short and
+// rows are many: 40000 x 64, 1 token 7.9 us on 64 x 64 tiles, 12.4 on 32 x 16).  Between
+// equals the smaller tile, which has more of the device at work.
+enum class ShortTile { k64, kWave32x16, kWave32x32, kGroup32x64, kGroup64x128 };
+
+inline ShortTile short_tile(long long rows, int tokens, int k, bool paired, bool residual, int cus) {
+  const long long kt = k / 64;
+  const long long end64 = residual ? 30 * (tokens < 32 ? tokens : 32) : 0;
+  const long long end128 = residual ? 14 * (tokens < 64 ? tokens : 64) : 0;
+  auto rounds = [&](int tn, int tt) { return rounds_of((rows + tn - 1) / tn * ((tokens + tt - 1) / tt), cus); };
+  auto wave = [&](int tn, int tt) { return rounds(tn, tt) * (1900 + (rounds(tn, tt) == 1 ? 100 : 160) * kt); };
+  ShortTile best = ShortTile::kWave32x16;
+  long long cost = wave(32, 16);
+  auto take = [&](ShortTile t, long long c) {
+    if (c < cost) {
+      best = t;
+      cost = c;
+    }
+  };
+  take(ShortTile::kWave32x32, wave(32, 32));
+  if (!paired) take(ShortTile::kGroup32x64, rounds(32, 64) * (1900 + 230 * kt));
+  take(ShortTile::k64, rounds(64, 64) * (1700 + end64 + 330 * kt));
+  take(ShortTile::kGroup64x128, rounds(64, 128) * (1900 + end128 + 420 * kt));
+  return best;
+}
+
 }  // namespace qd

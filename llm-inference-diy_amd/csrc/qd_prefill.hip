@@ -1566,36 +1566,14 @@ static GemmTile pick_tile(const BatchedGemvParams& p, int rows_per_out) {
   return 2 * mid >= cus && ring128_offsets32(p) ? GemmTile::k128 : GemmTile::k64;
 }
 
-// Products that would take the 64 x 64 tile: the shape by the time of its rounds
-// of workgroups, `cus` at a time.  Measured per round and K tile of 64 (us; cold
-// weights, n = 2048-11008 rows, K = 2048 and 5504): 64 x 64 0.29, 32 x 32 and 32 x 16
-// with K shared out over eight waves 0.12 for one round and 0.157 each for more,
-// 32 x 64 0.24 and 64 x 128 0.50 in two K groups.  Between equals the smaller tile,
-// which has more of the device at work.
-enum class ShortTile { k64, kWave32x16, kWave32x32, kGroup32x64, kGroup64x128 };
-
-static ShortTile pick_short(const BatchedGemvParams& p, int rows_per_out) {
-  // lane offsets stay below 2^31 (rows of 128 tokens or 64 weights past a workgroup's base)
+// Products that would take the 64 x 64 tile: short_tile's choice, where the lane offsets
+// stay below 2^31 (rows of 128 tokens or 64 weights past a workgroup's base) and the
+// grid below 2^20.
+static ShortTile pick_short(const BatchedGemvParams& p, int epi) {
   if (p.ldx >= (1LL << 23) || p.k >= (1 << 23)) return ShortTile::k64;
-  const long long cus = device_cus();
-  const long long rows = (long long)p.n * rows_per_out;
-  auto tiles = [&](int tn, int tt) { return (rows + tn - 1) / tn * ((p.t + tt - 1) / tt); };
-  if (tiles(32, 16) >= (1 << 20)) return ShortTile::k64;
-  auto rounds = [&](int tn, int tt) { return (tiles(tn, tt) + cus - 1) / cus; };
-  auto wave = [&](int tn, int tt) { return rounds(tn, tt) == 1 ? 120 : 157 * rounds(tn, tt); };
-  ShortTile best = ShortTile::kWave32x16;
-  long long cost = wave(32, 16);
-  auto take = [&](ShortTile t, long long c) {
-    if (c < cost) {
-      best = t;
-      cost = c;
-    }
-  };
-  take(ShortTile::kWave32x32, wave(32, 32));
-  if (rows_per_out == 1) take(ShortTile::kGroup32x64, 240 * rounds(32, 64));
-  take(ShortTile::k64, 290 * rounds(64, 64));
-  take(ShortTile::kGroup64x128, 500 * rounds(64, 128));
-  return best;
+  const long long rows = (long long)p.n * (epi == 3 ? 2 : 1);
+  if ((rows + 31) / 32 * ((p.t + 15) / 16) >= (1 << 20)) return ShortTile::k64;
+  return short_tile(rows, p.t, p.k, epi == 3, epi == 1, device_cus());
 }
 
 template <int NB, int TB, int W, int S, int kEpi>
@@ -1614,7 +1592,7 @@ static void launch_kgroup(const BatchedGemvParams& p, hipStream_t stream) {
 
 template <int kEpi>
 static hipError_t launch_short(const BatchedGemvParams& p, hipStream_t stream) {
-  switch (pick_short(p, kEpi == 3 ? 2 : 1)) {
+  switch (pick_short(p, kEpi)) {
     case ShortTile::kWave32x16: launch_wavek<2, 1, 8, 3, kEpi>(p, stream); break;
     case ShortTile::kWave32x32: launch_wavek<2, 2, 8, 2, kEpi>(p, stream); break;
     case ShortTile::kGroup32x64:

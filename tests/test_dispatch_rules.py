@@ -16,6 +16,9 @@ int shares_fused(int heads, int seqlen, int tokens, int cus) { return qd::prefil
 int shares_split(int heads, int seqlen, int tokens, int cus) { return qd::prefill_shares_split(heads, seqlen, tokens, cus); }
 int merges_by_wave(int heads, int tokens, int splits) { return qd::prefill_merges_by_wave(heads, tokens, splits); }
 int exact_two_rows(int tokens, int n, int k, int cus) { return qd::exact_two_rows(tokens, n, k, cus); }
+int short_tile(long long rows, int tokens, int k, int paired, int res, int cus) {
+  return (int)qd::short_tile(rows, tokens, k, paired, res, cus);
+}
 }
 """
 
@@ -77,3 +80,22 @@ def test_prompt_merge_takes_the_faster_form(rules, heads, tokens, splits, group_
     (4, 2048, 5504, 10.6, 11.3), (6, 2048, 5504, 12.7, 11.2), (16, 2048, 2048, 10.4, 6.2)])
 def test_exact_product_takes_the_faster_kernel(rules, tokens, n, k, two_rows_us, matrix_us):
     assert bool(rules.exact_two_rows(tokens, n, k, CUS)) == (two_rows_us < matrix_us)
+
+
+@pytest.mark.parametrize("tokens,n,k,paired,res,us", [   # 64 x 64, 32 x 16, 32 x 32, 32 x 64, 64 x 128
+    (1, 40000, 64, 0, 0, (7.86, 12.43, 12.60, 12.95, 10.23)), (32, 20000, 128, 0, 0, (7.01, 12.74, 8.88, 8.86, 8.05)),
+    (1, 20000, 512, 0, 0, (9.12, 10.14, 10.34, 10.64, 10.90)), (16, 40000, 512, 0, 0, (15.28, 18.60, 18.75, 20.22, 18.07)),
+    (1, 10000, 512, 1, 0, (9.06, 10.83, 10.98, None, 11.52)), (16, 15000, 512, 1, 0, (11.00, 15.74, 15.84, None, 12.98)),
+    (1, 64, 2048, 0, 0, (9.33, 4.80, 5.29, 6.84, 11.35)), (16, 2048, 5504, 0, 0, (20.09, 9.47, 10.32, 13.17, 25.00)),
+    (100, 2048, 2048, 0, 0, (10.14, 9.47, 6.63, 7.73, 12.64)), (100, 6144, 2048, 0, 0, (10.99, 23.15, 15.26, 13.48, 12.86)),
+    (64, 6144, 2048, 0, 0, (10.34, 13.72, 11.79, 8.31, 12.64)), (32, 6144, 2048, 0, 0, (10.19, 10.21, 7.74, 7.79, 12.21)),
+    (100, 5504, 2048, 1, 0, (23.69, 47.51, 34.52, None, 18.38)), (100, 2048, 5504, 0, 0, (20.47, 15.86, 11.23, 14.04, 26.90)),
+    (127, 11008, 2048, 0, 0, (23.94, 56.21, 37.28, 28.45, 19.38)), (65, 40000, 2048, 0, 0, (68.11, 109.84, 78.89, 70.53, 47.15)),
+    (200, 1000, 2048, 1, 0, (10.72, 17.28, 11.38, None, 13.46)), (160, 2048, 1024, 0, 0, (7.05, 10.48, 8.59, 6.05, 8.98)),
+    (48, 1536, 512, 0, 0, (5.18, 4.11, 4.27, 4.60, 6.27)), (400, 1000, 1024, 0, 0, (7.13, 12.50, 8.14, 5.96, 8.88)),
+    (48, 6144, 64, 0, 1, (5.37, 7.71, 5.97, 4.32, 5.64)), (16, 20000, 512, 0, 1, (11.79, 10.48, 10.74, 10.98, 11.50)),
+    (32, 20000, 512, 0, 1, (14.91, 15.19, 11.08, 11.29, 12.34)), (127, 20000, 256, 0, 1, (20.34, 47.43, 26.96, 16.10, 13.15)),
+    (100, 2048, 5504, 0, 1, (22.97, 16.26, 11.54, 14.38, 28.60)), (256, 2048, 2048, 0, 1, (11.61, 17.70, 11.39, 8.07, 14.24))])
+def test_short_product_takes_the_fastest_tile(rules, tokens, n, k, paired, res, us):
+    took = us[rules.short_tile(ctypes.c_longlong(n * (1 + paired)), tokens, k, paired, res, CUS)]
+    assert took is not None and took <= 1.05 * min(t for t in us if t is not None)

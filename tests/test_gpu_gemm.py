@@ -281,6 +281,18 @@ def test_mfma_short_prompt_tiles(qdiy, m, n, k, form):
     assert np.all(np.abs(got - want) <= tol), float(np.max(np.abs(got - want) - tol))
 
 
+@pytest.mark.parametrize("m,n,k", [
+    # short K, where a round's fixed part decides: 64 x 64 tiles in one and several rounds,
+    # 32 x 64 tiles from two K tiles on, 64 x 128 tiles over many rows
+    (9, 20000, 64), (33, 8190, 128), (63, 6144, 128), (65, 20010, 256), (127, 11000, 64),
+    # one K tile: with a residual the 32 x 64 tile, whose second K group then has none
+    (63, 6144, 64), (50, 6000, 64)])
+@pytest.mark.parametrize("form", ["plain", "residual", "swiglu"])
+def test_mfma_short_prompt_tiles_short_k(qdiy, m, n, k, form):
+    """The tiles of the test above where K is short."""
+    test_mfma_short_prompt_tiles(qdiy, m, n, k, form)
+
+
 @pytest.mark.parametrize("m,n,k,ldy", [(37, 100, 512, 100), (127, 1368, 2048, 1368),
                                         # from 128 rows: the 64 x 64 tile (n = 130, a strided
                                         # output), the 128 x 128 ring tile (a ragged last tile at
