@@ -170,11 +170,19 @@ def _check(rc: int) -> None:
 # call does here is kept short: pointers and streams go to ctypes as plain ints, and
 # the current stream is read as a handle (0.3 us) instead of through a
 # torch.cuda.Stream object (3.0 us).  A decode attention's call takes 5.6 us of host
-# time, 9.2 with c_void_p objects and stream objects.
+# time, 9.2 with c_void_p objects and stream objects.  The two functions that give the
+# handle are torch's own internals: where a torch lacks one, the stream object serves.
+
+def _current_stream() -> int:
+    try:
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    except AttributeError:
+        return torch.cuda.current_stream().cuda_stream
+
 
 def _stream(stream) -> int:
     if stream is None:
-        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        return _current_stream()
     if isinstance(stream, torch.cuda.Stream):
         stream = stream.cuda_stream
     return int(stream)

@@ -165,3 +165,20 @@ def test_decode_ops_reject_overlapping_outputs_without_a_gpu(qdiy):
         assert lib.qd_lm_head_argmax(P(xs), P(nw), ctypes.c_float(1e-6), P(wl), P(lg), V, H, P(wk),
                                      ctypes.c_size_t(ws_n), P(tk), None) == qdiy.QD_EINVAL
         assert b"overlap" in lib.qd_last_error()
+
+
+@pytest.mark.parametrize("missing", ["_cuda_getCurrentRawStream", "_cuda_getDevice"])
+def test_current_stream_without_torch_internals(monkeypatch, missing):
+    """The default stream argument where this torch lacks a function that gives the handle,
+    and (both there) as that function's handle."""
+    import types
+
+    import torch
+    import qdiy
+    for name in ("_cuda_getCurrentRawStream", "_cuda_getDevice"):
+        monkeypatch.setattr(torch._C, name, lambda *a: 40 + len(a), raising=False)
+    assert qdiy._stream(None) == 41
+    monkeypatch.delattr(torch._C, missing)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=77))
+    assert qdiy._stream(None) == 77
+    assert qdiy._stream(5) == 5
