@@ -440,9 +440,8 @@ def test_engine_mfma_prefill(qdiy, hidden, inter, n_prompt):
     """MFMA prefill against exact prefill on the same prompt (with c_proj exact
     where inter is not a multiple of 64): the next step's logits agree to the
     fp32-order difference, and plain decode steps are bit-identical in both
-    modes.  At hidden 2048 and 299 tokens the o_proj and c_proj products have
-    48 tiles of 128 x 128 and run split over K on that tile (engine workspace,
-    then the fold launch); gate/up is one launch with the SwiGLU epilogue."""
+    modes.  Gate/up is one launch with the SwiGLU epilogue; at hidden 2048 and 299
+    tokens o_proj and c_proj share K out inside short tiles' workgroups."""
     cfg = qdiy.model_cfg(vocab_size=512, hidden_size=hidden, num_layers=2, num_heads=hidden // 128,
                          intermediate_size=inter, max_seqlen=n_prompt + 20)
     img = qdiy.random_model_image(cfg, 41 + hidden, 0.03, nthreads=8)
@@ -487,6 +486,33 @@ def test_engine_mfma_prefill(qdiy, hidden, inter, n_prompt):
         if layer == 0:
             k0 = kv[qdiy.GEMM_MFMA][0][0].astype(np.float64)
             assert np.mean(np.abs(k0 - bad_k[0]) > 4 * ulp16(np.max(np.abs(bad_k[0])))) > 0.3
+
+
+@pytest.mark.parametrize("inter,tokens", [(5504, 1024), (5440, 899), (64, 1000)])
+def test_engine_mfma_prefill_two_slices_of_k(qdiy, inter, tokens):
+    """Hidden 2048 with 897 to 1024 tokens: o_proj and c_proj have 128 tiles of 128 x 128,
+    half the compute units, and run as two slices of K with a fold launch.  86 K tiles; 85
+    (slices of 43 and 42) with 3 rows in the last token tile; a single one, which no slice can
+    share.  What the second layer's KV rows see of both products is no further from float64
+    than in the exact mode (the two differ by the order of fp32 sums alone)."""
+    cfg = qdiy.model_cfg(vocab_size=512, hidden_size=2048, num_layers=2, num_heads=16,
+                         intermediate_size=inter, max_seqlen=tokens + 8)
+    img = qdiy.random_model_image(cfg, 43 + inter, 0.03, nthreads=8)
+    prompt = [int(t) for t in np.random.default_rng(tokens).integers(0, 512, tokens)]
+    kv = {}
+    with qdiy.Engine(image=img) as eng:
+        for mode in (qdiy.GEMM_EXACT, qdiy.GEMM_MFMA):
+            eng.set_prefill_mode(mode)
+            eng.reset()
+            eng.prefill(prompt)
+            kv[mode] = [a.astype(np.float64) for a in eng.kv_rows(1, 0, tokens)]
+    ref_k, ref_v = model_kv_fp64(model_tensors(img), prompt)
+    for i, ref in enumerate((ref_k[1], ref_v[1])):
+        scale = np.max(np.abs(ref), axis=1, keepdims=True)
+        err = {mode: np.abs(kv[mode][i] - ref) for mode in kv}
+        assert np.all(err[qdiy.GEMM_MFMA] <= 0.01 * scale), float(np.max(err[qdiy.GEMM_MFMA] / scale))
+        rms = {mode: np.sqrt(np.mean(err[mode] ** 2, axis=1)) for mode in kv}     # per token
+        assert np.all(rms[qdiy.GEMM_MFMA] <= 2 * rms[qdiy.GEMM_EXACT])
 
 
 def test_engine_mfma_prefill_two_passes(qdiy):
