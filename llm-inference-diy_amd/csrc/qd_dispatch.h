@@ -74,9 +74,17 @@ inline bool prefill_merges_by_wave(int heads, int tokens, int splits) {
 // no prefetch and a CU to themselves, so it stays the faster one only while they all run
 // at once: 1 / 4 tokens, K = 7176, 1024 rows 8.2 / 11.9 against 13.0 / 12.9, 2048 rows
 // 9.7 / 13.4 against 14.3 / 14.1, 4096 rows 17.7 / 24.6 against 17.1 / 15.6.
+// With a few tokens more it is still ahead on both sides of the usual widths.  Up to 128
+// weight rows, K = 256 to 5632, the matrix kernel's few workgroups only wait: 5 tokens 98 x
+// 1928 5.4 against 6.0, 6 tokens 3 x 1416 4.1 and 4.8, but 5 tokens 176 x 3176 8.9 and 7.0.
+// Past one 32 x 32 tile per CU the matrix kernel's next round is not paid for where K is
+// short: 6 tokens 9997 x 240 5.6 and 6.8, 10219 x 936 8.9 and 10.0, but 6931 x 624 6.8 and
+// 6.0; 8 tokens 11530 x 440 7.0 and 8.0, but 11773 x 552 8.6 and 8.0.
 constexpr int kWideTwoRowWg = 8;   // weight rows per workgroup of the two-row kernel from K = 7169
 inline bool exact_two_rows(int tokens, int n, int k, int cus) {
-  if (tokens > 4) return false;
+  if (tokens > 8) return false;
+  if (tokens > 4 && n > 32 * cus) return tokens <= 6 ? k > 128 && k <= 1024 : k > 256 && k <= 512;
+  if (tokens > 4) return tokens <= 6 && n <= 128 && k > 256 && k <= 5632;
   return k <= 7168 || (n + kWideTwoRowWg - 1) / kWideTwoRowWg <= cus;
 }
 

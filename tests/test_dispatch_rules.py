@@ -77,7 +77,11 @@ def test_prompt_merge_takes_the_faster_form(rules, heads, tokens, splits, group_
     (1, 16, 8192, 6.55, 13.40), (4, 16, 8192, 11.34, 13.33), (1, 1024, 7176, 8.15, 13.03), (4, 2048, 7176, 13.36, 14.14),
     (1, 2048, 8192, 11.32, 15.79), (2, 2048, 7680, 10.49, 14.86), (1, 4096, 8192, 20.42, 17.64),
     (4, 4096, 7176, 24.55, 15.59), (5, 4096, 8192, 36.91, 16.91), (5, 2048, 7176, 16.19, 14.21), (4, 6144, 2048, 9.1, 10.3),
-    (4, 2048, 5504, 10.6, 11.3), (6, 2048, 5504, 12.7, 11.2), (16, 2048, 2048, 10.4, 6.2)])
+    (4, 2048, 5504, 10.6, 11.3), (6, 2048, 5504, 12.7, 11.2), (16, 2048, 2048, 10.4, 6.2),
+    (5, 98, 1928, 5.43, 6.02), (5, 6, 5400, 9.15, 10.15), (6, 3, 1416, 4.07, 4.79), (6, 90, 1352, 4.50, 4.76),
+    (5, 15, 304, 2.91, 2.98), (5, 176, 3176, 8.85, 7.00), (6, 10219, 936, 8.90, 10.04), (5, 11934, 416, 6.32, 8.08), (6, 6931, 624, 6.77, 6.04),
+    (6, 11228, 128, 5.74, 5.20), (5, 8488, 1296, 10.64, 10.33), (6, 9997, 240, 5.63, 6.76), (6, 12892, 1088, 12.31, 11.34),
+    (8, 11530, 440, 7.03, 7.97), (7, 23427, 504, 11.01, 12.48), (8, 11773, 552, 8.57, 7.96), (7, 11682, 8, 5.42, 4.31)])
 def test_exact_product_takes_the_faster_kernel(rules, tokens, n, k, two_rows_us, matrix_us):
     assert bool(rules.exact_two_rows(tokens, n, k, CUS)) == (two_rows_us < matrix_us)
 

@@ -160,6 +160,32 @@ def test_exact_mode_two_row_kernel(qdiy, m, k, with_res):
         assert _same(got[i, :n], want), f"row {i}"
 
 
+@pytest.mark.parametrize("m,n,k", [
+    # both sides of the two-row kernel's ranges: few weight rows, and more than 32 per CU
+    # (8192 at 256)
+    (5, 1, 264), (6, 128, 5632), (5, 128, 5640), (6, 129, 5632), (5, 77, 256), (7, 99, 1000),
+    (6, 8192, 264), (5, 8193, 136), (6, 8211, 1024), (5, 8193, 1032), (6, 8200, 128),
+    (8, 8193, 512), (7, 8203, 264), (8, 8193, 520), (7, 8193, 256), (9, 8193, 512)])
+@pytest.mark.parametrize("with_res", [False, True])
+def test_exact_mode_five_to_eight_tokens(qdiy, m, n, k, with_res):
+    """5 to 9 tokens on either kernel: every output bit for bit, nothing past a row."""
+    pad = 5
+    rng = np.random.default_rng(31 * m + n + k + with_res)
+    x, W, R = normal_f16(rng, (m, k)), normal_f16(rng, (n, k), 0.02), normal_f16(rng, (m, n + pad))
+    y = torch.full((m, n + pad), 9.0, dtype=torch.float16, device="cuda")
+    qdiy.gemm_nt(_dev(x.reshape(-1)), _dev(W.reshape(-1)), y.view(-1), m, n, k, ldy=n + pad,
+                 residual=_dev(R.reshape(-1)) if with_res else None, mode=qdiy.GEMM_EXACT)
+    torch.cuda.synchronize()
+    got = y.cpu().numpy()
+    assert np.all(got[:, n:] == 9.0)
+    for i in range(m):
+        if with_res:
+            want = oracle.proj_residual(x[i], W.reshape(-1), R[i, :n], n, k)
+        else:
+            want = oracle.gemv(x[i], W.reshape(-1), n, k, 0, oracle.ORDER_WAVE64)
+        assert _same(got[i, :n], want), f"row {i}"
+
+
 @pytest.mark.parametrize("n", [2048, 2049])
 def test_exact_mode_wide_rows_change_kernel(qdiy, n):
     """K > 7168: up to 2048 weight rows on the two-row kernel, more on the matrix
