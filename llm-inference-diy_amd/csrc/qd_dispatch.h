@@ -102,14 +102,21 @@ inline bool exact_two_rows(int tokens, int n, int k, int cus) {
 // 9.7 us without, 14.6 with; on 32 x 32 tiles 10.6 and 11.0).  The tiles so chosen are
 // 0.15% (with a residual 0.6%) slower than the best of the five on average; by the times
 // per K tile alone they were 1.3% and up to 71% (the start decides where K is short and
-// rows are many: 40000 x 64, 1 token 7.9 us on 64 x 64 tiles, 12.4 on 32 x 16).  Between
-// equals the smaller tile, which has more of the device at work.
+// rows are many: 40000 x 64, 1 token 7.9 us on 64 x 64 tiles, 12.4 on 32 x 16).  Where a
+// lane's four outputs cannot be stored together (`scalar`: y or its rows off 8 bytes), the
+// 64 x 128 tile ends later still, as its lanes hold tokens and the 64 x 64 tile's hold
+// adjacent outputs: 0.022 us per token of 128, 0.012 with a residual, nothing measurable
+// for a pair's half as many (1367 tokens 2010 x 64 13.8 us, 10.2 on 64 x 64 tiles; 403
+// 5123 x 448 17.2 and 14.8).  Over 360 such products of 6 us and more the choice is
+// then 0.5% (residual 0.7%) slower than the best tile on average, 4.1% (1.4%) without.
+// Between equals the smaller tile, which has more of the device at work.
 enum class ShortTile { k64, kWave32x16, kWave32x32, kGroup32x64, kGroup64x128 };
 
-inline ShortTile short_tile(long long rows, int tokens, int k, bool paired, bool residual, int cus) {
+inline ShortTile short_tile(long long rows, int tokens, int k, bool paired, bool residual, bool scalar, int cus) {
   const long long kt = k / 64;
   const long long end64 = residual ? 30 * (tokens < 32 ? tokens : 32) : 0;
-  const long long end128 = residual ? 14 * (tokens < 64 ? tokens : 64) : 0;
+  const long long per_token = paired || !scalar ? 0 : residual ? 12 : 22;
+  const long long end128 = (residual ? 14 * (tokens < 64 ? tokens : 64) : 0) + per_token * (tokens < 128 ? tokens : 128);
   auto rounds = [&](int tn, int tt) { return rounds_of((rows + tn - 1) / tn * ((tokens + tt - 1) / tt), cus); };
   auto wave = [&](int tn, int tt) { return rounds(tn, tt) * (1900 + (rounds(tn, tt) == 1 ? 100 : 160) * kt); };
   ShortTile best = ShortTile::kWave32x16;

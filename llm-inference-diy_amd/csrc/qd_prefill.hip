@@ -1552,10 +1552,13 @@ static bool ring128_offsets32(const BatchedGemvParams& p) {
   return (long long)(p.n + kRgN) * p.k * 2 < (1LL << 32) && (long long)(p.t + kRgT) * p.ldx * 2 < (1LL << 32);
 }
 
+// Four adjacent outputs (and residuals) can be accessed as one 8-byte word.
+static bool outputs_vec8(const BatchedGemvParams& p) {
+  return ((reinterpret_cast<uintptr_t>(p.y) | reinterpret_cast<uintptr_t>(p.res)) & 7u) == 0 && p.ldy % 4 == 0;
+}
+
 static GemmTile pick_tile(const BatchedGemvParams& p, int rows_per_out) {
-  const bool vec8 = ((reinterpret_cast<uintptr_t>(p.y) | reinterpret_cast<uintptr_t>(p.res)) & 7u) == 0 &&
-                    p.ldy % 4 == 0;
-  if (p.t < kRingMinRows || !vec8) return GemmTile::k64;
+  if (p.t < kRingMinRows || !outputs_vec8(p)) return GemmTile::k64;
   const int cus = device_cus();
   const long long big = (long long)((p.n * rows_per_out + kR2N - 1) / kR2N) * ((p.t + kR2T - 1) / kR2T);
   // the 192 x 256 tile's buffer loads take 32-bit byte offsets up to a tile past each operand's end
@@ -1573,7 +1576,7 @@ static ShortTile pick_short(const BatchedGemvParams& p, int epi) {
   if (p.ldx >= (1LL << 23) || p.k >= (1 << 23)) return ShortTile::k64;
   const long long rows = (long long)p.n * (epi == 3 ? 2 : 1);
   if ((rows + 31) / 32 * ((p.t + 15) / 16) >= (1 << 20)) return ShortTile::k64;
-  return short_tile(rows, p.t, p.k, epi == 3, epi == 1, device_cus());
+  return short_tile(rows, p.t, p.k, epi == 3, epi == 1, !outputs_vec8(p), device_cus());
 }
 
 template <int NB, int TB, int W, int S, int kEpi>

@@ -16,8 +16,8 @@ int shares_fused(int heads, int seqlen, int tokens, int cus) { return qd::prefil
 int shares_split(int heads, int seqlen, int tokens, int cus) { return qd::prefill_shares_split(heads, seqlen, tokens, cus); }
 int merges_by_wave(int heads, int tokens, int splits) { return qd::prefill_merges_by_wave(heads, tokens, splits); }
 int exact_two_rows(int tokens, int n, int k, int cus) { return qd::exact_two_rows(tokens, n, k, cus); }
-int short_tile(long long rows, int tokens, int k, int paired, int res, int cus) {
-  return (int)qd::short_tile(rows, tokens, k, paired, res, cus);
+int short_tile(long long rows, int tokens, int k, int paired, int res, int scalar, int cus) {
+  return (int)qd::short_tile(rows, tokens, k, paired, res, scalar, cus);
 }
 }
 """
@@ -101,5 +101,15 @@ def test_exact_product_takes_the_faster_kernel(rules, tokens, n, k, two_rows_us,
     (32, 20000, 512, 0, 1, (14.91, 15.19, 11.08, 11.29, 12.34)), (127, 20000, 256, 0, 1, (20.34, 47.43, 26.96, 16.10, 13.15)),
     (100, 2048, 5504, 0, 1, (22.97, 16.26, 11.54, 14.38, 28.60)), (256, 2048, 2048, 0, 1, (11.61, 17.70, 11.39, 8.07, 14.24))])
 def test_short_product_takes_the_fastest_tile(rules, tokens, n, k, paired, res, us):
-    took = us[rules.short_tile(ctypes.c_longlong(n * (1 + paired)), tokens, k, paired, res, CUS)]
+    took = us[rules.short_tile(ctypes.c_longlong(n * (1 + paired)), tokens, k, paired, res, 0, CUS)]
     assert took is not None and took <= 1.05 * min(t for t in us if t is not None)
+
+
+@pytest.mark.parametrize("tokens,n,k,paired,res,us", [   # the same tiles, y rows an odd number of elements apart
+    (1367, 2010, 64, 0, 0, (10.15, 46.75, 27.64, 19.76, 13.78)), (559, 7218, 128, 0, 0, (14.08, 68.30, 40.18, 25.78, 18.01)),
+    (231, 9978, 192, 0, 0, (11.61, 43.32, 28.64, 18.56, 14.61)), (403, 5123, 448, 0, 0, (14.77, 43.55, 27.18, 19.84, 17.18)),
+    (1375, 1722, 512, 0, 0, (14.96, 48.18, 30.32, 20.38, 17.17)), (34, 9182, 128, 0, 1, (6.39, 13.00, 10.50, 9.00, 8.85)),
+    (426, 5067, 64, 0, 1, (15.58, 45.41, 26.65, 20.14, 20.43)), (1301, 1901, 128, 0, 1, (16.89, 52.81, 29.97, 20.24, 20.25))])
+def test_short_product_with_unaligned_outputs_takes_the_fastest_tile(rules, tokens, n, k, paired, res, us):
+    took = us[rules.short_tile(ctypes.c_longlong(n * (1 + paired)), tokens, k, paired, res, 1, CUS)]
+    assert took <= 1.05 * min(us)

@@ -319,6 +319,13 @@ def test_mfma_short_prompt_tiles_short_k(qdiy, m, n, k, form):
     test_mfma_short_prompt_tiles(qdiy, m, n, k, form)
 
 
+@pytest.mark.parametrize("m,n,k", [(231, 9979, 192), (303, 8703, 64), (403, 5123, 448), (34, 9183, 128)])
+@pytest.mark.parametrize("form", ["plain", "residual", "swiglu"])
+def test_mfma_short_prompt_tiles_unaligned_rows(qdiy, m, n, k, form):
+    """Rows of y an odd number of elements apart: where that moves the choice of the tile."""
+    test_mfma_short_prompt_tiles(qdiy, m, n, k, form)
+
+
 @pytest.mark.parametrize("m,n,k,ldy", [(37, 100, 512, 100), (127, 1368, 2048, 1368),
                                         # from 128 rows: the 64 x 64 tile (n = 130, a strided
                                         # output), the 128 x 128 ring tile (a ragged last tile at
