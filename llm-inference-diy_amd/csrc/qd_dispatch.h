@@ -3,6 +3,8 @@
 // (tests/test_dispatch_rules.py).
 #pragma once
 
+#include <cstddef>
+
 namespace qd {
 
 constexpr int kPfQ = 16;   // queries per workgroup of prefill_exact_kernel
@@ -132,6 +134,20 @@ inline ShortTile short_tile(long long rows, int tokens, int k, bool paired, bool
   take(ShortTile::k64, rounds(64, 64) * (1700 + end64 + 330 * kt));
   take(ShortTile::kGroup64x128, rounds(64, 128) * (1900 + end128 + 420 * kt));
   return best;
+}
+
+// Whether a product on `tiles` 128 x 128 tiles, one workgroup and CU each, shares K out over
+// two slices, folded by a second launch: where both slices of every tile run at once.  That
+// tile is taken from half of the CUs on (pick_tile), so this is exactly half of them: 897-1024
+// tokens of 2048 rows, 385-512 of 4096, 1921-2048 of 1024.  Engine prompts, us a layer, one
+// slice / two: 128 tiles on 256 CUs 237.6 / 221.7 (hidden 2048, FFN 5504, 1022 tokens), 337.0
+// / 304.5 (4096, 8192, 510), 160.5 / 158.3 (2048, 2048); 144 tiles, where two slices take a
+// second round, 258.7 / 275.4 (1100 tokens); 120 tiles, by then on the short tiles, 237.0 /
+// 239.4 (1024, 8192, 1918), 231.3 / 237.4 (2560, 6912, 668).
+inline bool ring_two_slices(long long tiles, int cus) { return 2 * tiles <= cus; }
+// Bytes of the fp32 partials of two slices under that rule (16 MiB on 256 CUs).
+inline size_t ring_two_slice_bytes(int outputs_per_tile, int cus) {
+  return (size_t)(cus / 2) * 2 * outputs_per_tile * sizeof(float);
 }
 
 }  // namespace qd

@@ -253,7 +253,7 @@ int prefill_batched(qd_engine* e, const int* tokens, int T, int pos0) {
                   long long ldy, int epi) {
     qd::BatchedGemvParams p{x, ldx, w, n, k, T, y, ldy, y};
     if (e->prefill_mode == QD_GEMM_MFMA && k % 64 == 0)
-      return qd::launch_gemm_mfma_split(p, epi, e->p_split, qd::kGemmSplitWsBytes, e->stream);
+      return qd::launch_gemm_mfma_split(p, epi, e->p_split, e->stream);
     return qd::launch_gemv_batched(p, epi, e->stream);
   };
   for (uint32_t l = 0; l < c.num_layers && he == hipSuccess; ++l) {
@@ -523,7 +523,7 @@ int qd_engine_create_from_image(const void* image, long long bytes, qd_engine** 
       {(void**)&e->weights, wbytes},  {(void**)&e->k_cache, e->kv_bytes}, {(void**)&e->v_cache, e->kv_bytes},
       {(void**)&e->x, H * 2},         {(void**)&e->qkv, 3 * H * 2},     {(void**)&e->attn_out, H * 2},
       {(void**)&e->act, I * 2},       {(void**)&e->logits, V * 2},      {&e->lm_ws, (long long)e->lm_ws_bytes},
-      {(void**)&e->p_split, (long long)qd::kGemmSplitWsBytes}};
+      {(void**)&e->p_split, (long long)qd::gemm_split_ws_bytes()}};
   for (auto& a : allocs) {
     if ((he = hipMalloc(a.p, (size_t)a.n)) != hipSuccess) {
       engine_free(e);

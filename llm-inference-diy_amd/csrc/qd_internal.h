@@ -384,13 +384,11 @@ hipError_t launch_gemm_exact_mfma(const BatchedGemvParams& p, int epi, int cus, 
 // The same product on the matrix cores (fp32 accumulation in the hardware's
 // order, not bit-reproducible on the host); p.k must be a multiple of 64.
 hipError_t launch_gemm_mfma(const BatchedGemvParams& p, int epi, hipStream_t stream);
-// The same, allowed to split K over two slices when the tile grid leaves half of
-// the CUs idle: fp32 partial sums in `workspace`, then one launch folds them in
-// slice order and applies the epilogue.
-// Otherwise, and without a workspace, it is launch_gemm_mfma.
-constexpr size_t kGemmSplitWsBytes = (size_t)64 << 20;
-hipError_t launch_gemm_mfma_split(const BatchedGemvParams& p, int epi, float* workspace,
-                                  size_t workspace_bytes, hipStream_t stream);
+// The same, sharing K out over two slices where its tiles leave half of the CUs idle
+// (ring_two_slices): fp32 partial sums in `workspace`, gemm_split_ws_bytes() of it, then
+// one launch folds them in slice order and applies the epilogue.
+size_t gemm_split_ws_bytes();
+hipError_t launch_gemm_mfma_split(const BatchedGemvParams& p, int epi, float* workspace, hipStream_t stream);
 // act[t][i] = half(g * (u / (1 + exp(-u)))) with g = half(X W1^T), u = half(X W2^T)
 // (p.w = W1, p.w2 = W2, p.n = inter, p.y = act) in one matrix-core launch, the
 // SwiGLU applied in the GEMM's epilogue: from 128 tokens (act 8-byte aligned,

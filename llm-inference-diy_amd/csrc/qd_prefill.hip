@@ -553,18 +553,16 @@ __global__ __launch_bounds__(256) void gemm_nt_mfma_kernel(BatchedGemvParams p) 
     }
 }
 
-// Folds the split-K partials of gemm_nt_ring128_kernel<2>: the slices' fp32 sums
+// Folds the split-K partials of gemm_nt_ring128_kernel<2>: the two slices' fp32 sums
 // added in slice order, then the epilogue of kEpi (0: half(sum); 1: half(R +
 // half(sum))).  One thread per output.
 template <int kEpi>
-__global__ __launch_bounds__(256) void splitk_fold_kernel(BatchedGemvParams p, int splits) {
+__global__ __launch_bounds__(256) void splitk_fold_kernel(BatchedGemvParams p) {
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   const long long tn = (long long)p.t * p.n;
   if (i >= tn) return;
-  float s = p.part[i];
-  for (int z = 1; z < splits; ++z) s += p.part[z * tn + i];
   const long long t = i / p.n, n = i - t * p.n;
-  _Float16 y = to_f16(s);
+  _Float16 y = to_f16(p.part[i] + p.part[tn + i]);
   if constexpr (kEpi == 1) y = (_Float16)((float)reinterpret_cast<const _Float16*>(p.res)[t * p.ldy + n] + (float)y);
   reinterpret_cast<_Float16*>(p.y)[t * p.ldy + n] = y;
 }
@@ -1655,40 +1653,31 @@ hipError_t launch_gemm_mfma_swiglu(const BatchedGemvParams& p, hipStream_t strea
   return hipGetLastError();
 }
 
-// Where the product takes 128 x 128 tiles and they fill at most half of the
-// device (1023 tokens of 2048 rows: 128 tiles), splits K over two slices of whole
-// 64-wide tiles when n is a multiple of 4 and the workspace holds the slices' fp32
-// partials; one launch then adds them in order with the epilogue
-// (splitk_fold_kernel): a 1023-token matrix-core prompt of 24 layers 5.13 ms
-// against 5.49 unsplit.  Fewer tokens share K out inside a workgroup
-// (launch_short), with no second launch: prompts of 127 / 255 / 511 / 800 tokens
-// 1.72 / 2.23 / 3.39 / 4.40 ms, split 2.02 / 2.66 / 3.85 / 5.01.
-hipError_t launch_gemm_mfma_split(const BatchedGemvParams& p, int epi, float* workspace,
-                                  size_t workspace_bytes, hipStream_t stream) {
+size_t gemm_split_ws_bytes() { return ring_two_slice_bytes(kRgN * kRgT, device_cus()); }
+
+// As launch_gemm_mfma, but where the 128 x 128 tiles leave half of the device idle
+// (ring_two_slices) K is shared out over two slices of whole 64-wide tiles when n is a
+// multiple of 4; one launch then adds their fp32 partials in order with the epilogue
+// (splitk_fold_kernel).  Fewer tokens share K out inside a workgroup (launch_short), with
+// no second launch: prompts of 127 / 255 / 511 / 800 tokens 1.72 / 2.23 / 3.39 / 4.40 ms,
+// split 2.02 / 2.66 / 3.85 / 5.01.
+hipError_t launch_gemm_mfma_split(const BatchedGemvParams& p, int epi, float* workspace, hipStream_t stream) {
   if (p.k < 64 || p.k % 64 != 0 || p.t < 1 || p.n < 1) return hipErrorInvalidValue;
   const long long tiles = (long long)((p.n + kRgN - 1) / kRgN) * ((p.t + kRgT - 1) / kRgT);
-  int splits = workspace && pick_tile(p, 1) == GemmTile::k128 && p.n % 4 == 0 && 2 * tiles <= device_cus() ? 2 : 1;
-  if (splits > 1) {
-    // slices of whole K tiles, none empty, as many as the workspace holds
-    while (splits > 1 && (size_t)splits * p.t * p.n * sizeof(float) > workspace_bytes) --splits;
-    const int kslice = ((p.k + splits - 1) / splits + kMmK - 1) / kMmK * kMmK;
-    splits = (p.k + kslice - 1) / kslice;
-    if (splits > 1) {
-      BatchedGemvParams q = p;
-      q.part = workspace;
-      q.kslice = kslice;
-      hipLaunchKernelGGL(gemm_nt_ring128_kernel<2>, dim3((unsigned)tiles, splits), dim3(256), 0, stream, q);
-      hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return e;
-      const dim3 fgrid((unsigned)(((long long)p.t * p.n + 255) / 256));
-      if (epi == 0)
-        hipLaunchKernelGGL(splitk_fold_kernel<0>, fgrid, dim3(256), 0, stream, q, splits);
-      else
-        hipLaunchKernelGGL(splitk_fold_kernel<1>, fgrid, dim3(256), 0, stream, q, splits);
-      return hipGetLastError();
-    }
-  }
-  return launch_gemm_mfma(p, epi, stream);
+  if (p.k <= kRgK || p.n % 4 != 0 || pick_tile(p, 1) != GemmTile::k128 || !ring_two_slices(tiles, device_cus()))
+    return launch_gemm_mfma(p, epi, stream);
+  BatchedGemvParams q = p;
+  q.part = workspace;
+  q.kslice = (p.k / kRgK + 1) / 2 * kRgK;
+  hipLaunchKernelGGL(gemm_nt_ring128_kernel<2>, dim3((unsigned)tiles, 2), dim3(256), 0, stream, q);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const dim3 fgrid((unsigned)(((long long)p.t * p.n + 255) / 256));
+  if (epi == 0)
+    hipLaunchKernelGGL(splitk_fold_kernel<0>, fgrid, dim3(256), 0, stream, q);
+  else
+    hipLaunchKernelGGL(splitk_fold_kernel<1>, fgrid, dim3(256), 0, stream, q);
+  return hipGetLastError();
 }
 
 hipError_t launch_embed(const uint16_t* wte, const int* tokens, uint16_t* x, int hidden, int T,

@@ -19,6 +19,8 @@ int exact_two_rows(int tokens, int n, int k, int cus) { return qd::exact_two_row
 int short_tile(long long rows, int tokens, int k, int paired, int res, int scalar, int cus) {
   return (int)qd::short_tile(rows, tokens, k, paired, res, scalar, cus);
 }
+int ring_two_slices(long long tiles, int cus) { return qd::ring_two_slices(tiles, cus); }
+long long ring_two_slice_bytes(int outputs, int cus) { return (long long)qd::ring_two_slice_bytes(outputs, cus); }
 }
 """
 
@@ -113,3 +115,21 @@ def test_short_product_takes_the_fastest_tile(rules, tokens, n, k, paired, res, 
 def test_short_product_with_unaligned_outputs_takes_the_fastest_tile(rules, tokens, n, k, paired, res, us):
     took = us[rules.short_tile(ctypes.c_longlong(n * (1 + paired)), tokens, k, paired, res, 1, CUS)]
     assert took <= 1.05 * min(us)
+
+
+@pytest.mark.parametrize("n,tokens,one_us,two_us", [   # us a layer of the whole prompt, both products so
+    (2048, 1022, 237.6, 221.7), (4096, 510, 337.0, 304.5), (1024, 2046, 264.3, 247.9), (2048, 1100, 258.7, 275.4),
+    (2048, 1300, 285.5, 306.1), (2048, 1920, 303.3, 330.3)])
+def test_two_slices_of_k_where_both_run_at_once(rules, n, tokens, one_us, two_us):
+    tiles = -(-n // 128) * -(-tokens // 128)
+    assert bool(rules.ring_two_slices(ctypes.c_longlong(tiles), CUS)) == (two_us < one_us)
+
+
+@pytest.mark.parametrize("cus", [256, 255, 304, 64])
+def test_two_slices_of_k_fit_their_workspace(rules, cus):
+    rules.ring_two_slice_bytes.restype = ctypes.c_longlong
+    have = rules.ring_two_slice_bytes(128 * 128, cus)
+    for wide in range(1, cus + 1):
+        for high in range(1, cus // wide + 1):
+            if rules.ring_two_slices(ctypes.c_longlong(wide * high), cus):
+                assert 2 * (128 * wide) * (128 * high) * 4 <= have
