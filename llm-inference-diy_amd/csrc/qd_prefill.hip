@@ -579,10 +579,11 @@ constexpr int kRingMinRows = 128;            // the ring tiles from this many to
 // Why: on gemm_nt_mfma_kernel's 64 x 64 tiles a 2048-row product of a short prompt
 // has 32 or 64 workgroups, each a chain of K / 64 barrier steps of ~0.24 us,
 // weights in L2 or not; 32 x 32 and 32 x 16 tiles have a workgroup for every CU and
-// eight chains in each.  What bounds them is the bytes each CU takes in: ~0.7 MB
-// per CU at 67 GB/s for K = 5504.  Cold weights, 100 tokens: 2048 x 2048 10.9 ->
-// 6.2 us, 2048 x 5504 26.5 -> 13.1; 16 tokens: 9.9 -> 5.6, 21.2 -> 13.3, 6144 x
-// 2048 10.3 -> 7.9 us.
+// eight chains in each.  What bounds them is the wait for loads: at K = 5504, 100 tokens
+// 12.3 TB/s from L2 over the device with 128 KB per CU in flight, 48 GB/s a CU
+// (its direct loads reach ~150; the 128 x 128 tile takes 14.2 TB/s).  Cold weights,
+// 100 tokens: 2048 x 2048 10.9 -> 6.2 us, 2048 x 5504 26.5 -> 13.1; 16 tokens: 9.9
+// -> 5.6, 21.2 -> 13.3, 6144 x 2048 10.3 -> 7.9 us.
 template <int NB, int TB, int W, int S, int kEpi>
 __global__ __launch_bounds__(64 * W, W / 4) void gemm_nt_wavek_kernel(BatchedGemvParams p) {
   constexpr int kN = 16 * NB, kT = 16 * TB;             // rows of the W tile, tokens
