@@ -173,16 +173,12 @@ def _check(rc: int) -> None:
 # time, 9.2 with c_void_p objects and stream objects.  The two functions that give the
 # handle are torch's own internals: where a torch lacks one, the stream object serves.
 
-def _current_stream() -> int:
-    try:
-        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
-    except AttributeError:
-        return torch.cuda.current_stream().cuda_stream
-
-
 def _stream(stream) -> int:
     if stream is None:
-        return _current_stream()
+        try:
+            return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+        except AttributeError:
+            return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, torch.cuda.Stream):
         stream = stream.cuda_stream
     return int(stream)
