@@ -18,8 +18,8 @@
 //   rmsnorm_batched_kernel     T waves: xn[t] = RMSNorm(x[t]) * w
 //   gemm_exact_mfma_kernel     Y[t][n] = sum_k X[t][k] W[n][k], with an epilogue
 //                              (store as half, or residual add into the stream)
-//   gemv_batched_kernel        the same for up to 4 tokens (exact_two_rows): each weight row is
-//                              read once and kept in registers
+//   gemv_batched_kernel        the same for a few tokens (exact_two_rows): each
+//                              weight row is read once and kept in registers
 //   rope_batched_kernel        bias + RoPE + KV append per token (qd_rope_cache)
 //   swiglu_batched_kernel      act = half(g * (u / (1 + exp(-u))))
 // Attention runs per token with qd_decode_attention's plan for that length.
